@@ -108,6 +108,18 @@ int esp_dense_tile(const void* x, int x_dtype, int64_t x_stride, int64_t T, int6
                    int64_t xh_numel, float* Z, int64_t z_numel, int32_t* counters, int64_t counters_numel, int64_t k2,
                    int64_t cb, int64_t SK, void* stream);
 
+/* dense over a prompt of any number of rows with every weight decoded once (no reference counterpart): the rows rotated
+ * into xh and the weights decoded to fp16 into wf, then a GEMM on those fragments whose sums keep the order of a launch
+ * with K splits SK and KW k slots: the bits of esp_dense at that SK and W = 4 * KW, or of esp_dense_tile at that SK
+ * with KW = 2. x, the matrices and y as esp_dense_tile; xh fp16 scratch (xh_numel >= n_shards * ceil(T / 16) * 16 * K);
+ * wf fp16 scratch (wf_numel >= K * sum(n_cols)); SK * KW <= K / 32, KW 1 to 4. Alignment as esp_dense_tile, wf 16-byte
+ * aligned. */
+int esp_dense_prompt(const void* x, int x_dtype, int64_t x_stride, int64_t T, int64_t K, int64_t n_shards,
+                     const void* const* trellis, const void* const* suh, const void* const* svh, const int64_t* n_cols,
+                     const int64_t* col0, void* y, int y_dtype, int64_t y_stride, int64_t y_cols, void* xh,
+                     int64_t xh_numel, void* wf, int64_t wf_numel, int64_t k2, int64_t cb, int64_t SK, int64_t KW,
+                     void* stream);
+
 /* Replaces `route_group` (experts.cpp:214-223, route.cu:35-207): router logits x @ gate^T (+ the shared gate), top-k
  * by the exactly rounded bf16 logits (lowest id on ties), weights renormalised over the picks, the shared slot's
  * weight sigmoid(x . sgate), then the grouping of the picks. x [R][x_stride] and gate [E][H] in one dtype (bf16 or

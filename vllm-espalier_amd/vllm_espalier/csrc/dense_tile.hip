@@ -15,7 +15,7 @@
 // fixed step order, never on the other rows of the prompt or its place in a tile.
 #include <type_traits>
 
-#include "dense.hpp"
+#include "tile.hpp"
 
 namespace esp {
 
@@ -24,8 +24,6 @@ constexpr int TILE_RG = TILE_ROWS / 16;         // row groups a workgroup
 constexpr int TILE_WAVES = 8;                   // 4 pairs x 2 k slots
 constexpr int TILE_KW = TILE_WAVES / 4;
 constexpr int TILE_STEPS = 4;                   // 32-k steps a stage
-constexpr int TILE_FRAG = 512;                  // halves a (row group, step) block: 64 lanes x 8
-constexpr int RED_STRIDE = 132;                 // floats between two rows of the block's sums (banks apart)
 constexpr int RED_BYTES = TILE_ROWS * RED_STRIDE * 4;
 
 #ifdef ESP_PHASE_TRACE
@@ -105,35 +103,17 @@ __device__ __forceinline__ void tile_all_arrived(int* counter, int* seen, int to
     __syncthreads();
 }
 
-// xh of tile_rot_kernel: a workgroup takes one matrix, one row group of 16 rows and one 128-chunk of K, which fill
-// exactly the 4 (row group, step) A blocks of that chunk: a 32-lane half rotates 2 rows (rows past T are zero) into
-// their fragment places in shared memory, then the 4 KiB go out as one 16-byte store a thread, contiguous in xh
+// xh, a (matrix, row group, 128-chunk) a workgroup
 __global__ __launch_bounds__(256) void tile_rot_kernel(const void* __restrict__ x, int x_dtype, int x_stride, int T,
                                                        int K, int n, const uint16_t* suh0, const uint16_t* suh1,
                                                        const uint16_t* suh2, const uint16_t* suh3,
                                                        uint16_t* __restrict__ xh, int RG) {
     __shared__ __align__(16) uint16_t frag[4 * TILE_FRAG];
-    const int l32 = threadIdx.x & 31, hw = threadIdx.x >> 5;
-    const int nb = K >> 7;
-    const int ch = (int)(blockIdx.x % nb), rg = (int)((blockIdx.x / nb) % RG), s = (int)(blockIdx.x / (nb * RG));
-    const uint16_t* suh = s == 0 ? suh0 : s == 1 ? suh1 : s == 2 ? suh2 : suh3;
-    // the lane's 4 consecutive k (ch * 128 + 4 l32 ...) are 4 consecutive halves of one A fragment lane
-    const int kk = (4 * l32) & 31, kt = kk & 15;
-    const int sl = l32 >> 3;                                  // the step inside the chunk
-    const int G = 2 * (kk >> 4) + ((kt >> 2) & 1), hi = kt >> 3;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int rr = 2 * hw + i, r = rg * 16 + rr;
-        uint2 u = make_uint2(0u, 0u);
-        if (r < T) u = rot128(x, x_dtype, (size_t)r * x_stride + ch * 128, suh + ch * 128, l32);
-        *reinterpret_cast<uint2*>(frag + (sl * 64 + rr + 16 * G) * 8 + 4 * hi) = u;
-    }
-    __syncthreads();
-    uint16_t* dst = xh + (((size_t)s * RG + rg) * (K >> 5) + ch * 4) * TILE_FRAG;
+    int ch;
+    uint16_t* dst = tile_rot_unit(blockIdx.x, x, x_dtype, x_stride, T, K, suh0, suh1, suh2, suh3, xh, RG, frag, ch) +
+                    (size_t)ch * 4 * TILE_FRAG;              // the chunk's 4 KiB, one 16-byte store a thread
     reinterpret_cast<uint4*>(dst)[threadIdx.x] = reinterpret_cast<const uint4*>(frag)[threadIdx.x];
 }
-
-typedef __attribute__((address_space(3))) const f16x8* lds_f16x8_ptr;
 
 // The finisher's rows of one half-wave (rows rbase, rbase + 16, ...): RPB rows at a time with the other splits'
 // partials of those rows in flight together (RPB * OM loads, OM >= SK - 1), its own split's sums read from shared

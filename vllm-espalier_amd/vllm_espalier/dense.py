@@ -69,6 +69,13 @@ def tile_plan(K: int, N: int) -> int:
 
 
 TILE_ROWS = 128              # rows a prompt-launch workgroup
+TILE_SLOTS = 2               # k slots a workgroup of esp_dense_tile
+# From this many rows a prompt with decode's bits runs as esp_dense_prompt instead of windows of MAX_ROWS rows: 2 launches
+# and each weight decoded once, against a launch a window (config 2's four layers, MI355X: 114 us against 181 us at 128
+# rows; at 96, three windows, a K = 4096 layer alone would lose, 43 us against 39)
+PROMPT_MIN_ROWS = 97
+PROMPT_ROWS = 4096           # rows one esp_dense_prompt call takes (bounds its scratch)
+PROMPT_WEIGHTS = 1 << 27     # weights a launch decodes whole (2 bytes each)
 # launches whose last K split can poll the others' partials run as esp_dense_own over an all-ones partials buffer (the
 # same bits, no arrival count); ESPALIER_DENSE_OWN=0 runs every launch as esp_dense
 OWN = env("ESPALIER_DENSE_OWN", "1") != "0"
@@ -237,6 +244,43 @@ class Dense:
                 [self.col0[i] for i in pick], y, xh, zl, self.counters, l.k2, l.cb, l.sk, l.w, l.pf, ROT_SMEM)
         return y
 
+    def prompts(self) -> bool:
+        """Whether forward_prompt takes this layer: 128-wide blocks, and no launch with too many weights to decode
+        whole or with a K split shorter than its k slots."""
+        return (self.K % 128 == 0 and all(m.out_features % 128 == 0 for m in self.mats) and
+                all(self.K * l.n <= PROMPT_WEIGHTS and l.sk * (l.w // 4) <= self.K // 32 for l in self.launches))
+
+    def _tile_decodes_once(self, T: int, launch) -> bool:
+        """Whether T rows of a launch in the tile mode run as esp_dense_prompt (the bits of esp_dense_tile, every weight
+        decoded once): where esp_dense_tile's grid is past two 8-wave workgroups a CU, so its tiles decode the weights
+        again in a second round and its splits' partials follow one another (2048 -> 5120 at 509 / 1024 / 2048 rows: 40
+        / 70 / 125 us against 38 / 48 / 76; 4096 -> 2048: 33 / 59 / 105 against 41 / 42 / 57)."""
+        sk = tile_plan(self.K, launch.n)
+        return (-(-T // TILE_ROWS) * (launch.n // 128) * sk > 512 and self.K * launch.n <= PROMPT_WEIGHTS and
+                sk * TILE_SLOTS <= self.K // 32)
+
+    def _prompt(self, x, codes, pre, post, y, launch, sk: int, slots: int) -> None:
+        pick = launch.members
+        for r0 in range(0, x.shape[0], PROMPT_ROWS):
+            rows = slice(r0, r0 + PROMPT_ROWS)
+            ext().dense_prompt(x[rows], [codes[i] for i in pick], [pre[i] for i in pick], [post[i] for i in pick],
+                               [self.col0[i] for i in pick], y[rows], launch.k2, launch.cb, sk, slots)
+
+    def forward_prompt(self, x, trellis=None, suh=None, svh=None, out=None):
+        """x [T, K], any T (a prompt) -> [T, n_out] in x's dtype, with forward's bits a row and every weight decoded once
+        (esp_dense_prompt; only when prompts()). trellis / suh / svh as in forward."""
+        codes = trellis or [m.trellis for m in self.mats]
+        pre = suh or [m.suh for m in self.mats]
+        post = svh or [m.svh for m in self.mats]
+        y = torch.empty((x.shape[0], self.n_out), dtype=x.dtype, device=x.device) if out is None else out
+        if self.n_out > self.N:
+            y[:, self.N:].zero_()
+        if x.stride(-1) != 1:
+            x = x.contiguous()
+        for l in self.launches:
+            self._prompt(x, codes, pre, post, y, l, l.sk, l.w // 4)
+        return y
+
     def reserve_prompt(self, T: int) -> None:
         """Grow the prompt scratch for forward_tile over T rows (done before a graph is captured)."""
         device = self.mats[0].trellis.device
@@ -248,7 +292,7 @@ class Dense:
 
     def forward_tile(self, x, trellis=None, suh=None, svh=None, out=None):
         """x [T, K], any T (a prompt) -> [T, n_out] in x's dtype, each weight decoded once for every 128 rows
-        (esp_dense_tile). A row's bits are its own (the same at any T), not those of forward. trellis / suh / svh:
+        (esp_dense_tile) or once (esp_dense_prompt, the same bits). A row's bits are its own (the same at any T), not those of forward. trellis / suh / svh:
         lists that replace the matrices' own tensors, as in forward."""
         codes = trellis or [m.trellis for m in self.mats]
         pre = suh or [m.suh for m in self.mats]
@@ -259,13 +303,18 @@ class Dense:
             y[:, self.N:].zero_()
         if x.stride(-1) != 1:
             x = x.contiguous()
-        self.reserve_prompt(T)
+        if not all(self._tile_decodes_once(T, l) for l in self.launches):
+            self.reserve_prompt(T)
         z, xh, cnt = prompt_scratch(x.device, 0, 0, 0)
         e = ext()
         for l in self.launches:
             pick = l.members
+            sk = tile_plan(self.K, l.n)
+            if self._tile_decodes_once(T, l):
+                self._prompt(x, codes, pre, post, y, l, sk, TILE_SLOTS)
+                continue
             e.dense_tile(x, [codes[i] for i in pick], [pre[i] for i in pick], [post[i] for i in pick],
-                         [self.col0[i] for i in pick], y, xh, z, cnt, l.k2, l.cb, tile_plan(self.K, l.n))
+                         [self.col0[i] for i in pick], y, xh, z, cnt, l.k2, l.cb, sk)
         return y
 
     def norm_fusable(self, M: int) -> bool:
