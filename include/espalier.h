@@ -203,6 +203,21 @@ int esp_grouped_list(const void* X0, const void* X1, const int64_t* TP0, const i
                      int64_t z_numel, int64_t mats, int64_t K, int64_t N, int64_t P, int64_t SK, int64_t slots,
                      int64_t warps, int64_t lo, int64_t hi, void* stream);
 
+/* esp_tile_list for tiles of `rows` members (32 or 64): ceil(maxm / rows) and ceil(P / rows) in its bounds. */
+int esp_tile_list_rows(const int32_t* ucount, const int32_t* members, int64_t nexp_max, int64_t maxm, int64_t P,
+                       int64_t rows, int32_t* tiles, int64_t tiles_numel, void* stream);
+
+/* The expert GEMMs of a whole prompt over esp_tile_list_rows's list for tiles of tile_rows members (no reference
+ * counterpart): an expert's weights decoded once a tile and matrix, every split's scaled sums added in split order in
+ * the launch, so Z [mats][P][N] holds what esp_grouped's readers make of its [mats][SK][P][N] at SK splits and one wave
+ * of k slots (4 waves a workgroup), bit for bit. K and N multiples of 128, P * K < 2^31. Status bits as esp_grouped and
+ * esp_grouped_list. */
+int esp_grouped_prompt(const void* X0, const void* X1, const int64_t* TP0, const int64_t* TP1, const int32_t* B0,
+                       const int32_t* B1, const int32_t* C0, const int32_t* C1, const int32_t* uids, int64_t nexp_max,
+                       const int32_t* ucount, const int32_t* members, int64_t maxm, const int32_t* tiles,
+                       int64_t tile_rows, float* Z, int64_t z_numel, int64_t mats, int64_t K, int64_t N, int64_t P,
+                       int64_t SK, int64_t slots, int64_t lo, int64_t hi, void* stream);
+
 /* Replaces `gateup_epilogue` (experts.cpp:106-118, experts.cu:120-162, 477-487): per valid pick p, the gate / up
  * splits of Z [2][SK][P][N] summed in order, H, * svh, SwiGLU (act_mode 1: fp32; 0: bf16 roundings; clamped to
  * limit), * suh_d, H -> xd fp16 [P][N]. svh_g/svh_u/suh_d fp16 [E][N]. */

@@ -212,3 +212,20 @@ def test_status_bits_match_the_header():
     text = (Path(__file__).resolve().parent.parent / "include" / "espalier.h").read_text()
     bits = {int(v) for v in re.findall(r"^#define ESP_STATUS_\w+ (\d+)", text, re.M)}
     assert bits == {b for b, _ in X.STATUS_BITS}
+
+
+@pytest.mark.parametrize("rows", [32, 64])
+def test_tile_list_cap_of_taller_tiles(rows):
+    """tile_list_cap bounds the non-empty tiles of `rows` members of random and piled groupings."""
+    import random
+    from vllm_espalier import experts as X
+    rng = random.Random(rows)
+    for _ in range(200):
+        E, T, k = rng.randint(1, 300), rng.randint(1, 700), rng.randint(1, 8)
+        counts = [0] * E
+        for _ in range(T):
+            for e in rng.sample(range(E), min(k, E)) if rng.random() < 0.7 else list(range(min(k, E))):
+                counts[e] += 1
+        used = [c for c in counts if c]
+        tiles = sum(-(-c // rows) for c in used)
+        assert tiles <= X.tile_list_cap(min(T * k, E), T, T * k, rows)

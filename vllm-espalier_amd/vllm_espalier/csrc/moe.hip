@@ -1055,7 +1055,7 @@ __global__ __launch_bounds__(256) void down_combine_rows_kernel(const float* __r
 
 // ------------------------------------------------------------------------------------------------------------------
 // esp_tile_list: the non-empty (expert slot u, member tile t) pairs of a grouping, in (u, t) order, for
-// esp_grouped_list: tiles[0] = their number, tiles[1 + i] = u << 16 | t. A tile is non-empty iff its first member is
+// esp_grouped_list (tiles of 32 members) and esp_grouped_prompt (32 or 64): tiles[0] = their number, tiles[1 + i] = u << 16 | t. A tile is non-empty iff its first member is
 // (members come first in a row, -1 padded). One workgroup: each thread tests its run of consecutive pairs with every
 // load in flight, then a block-wide prefix of the counts places the entries. At most cap entries are written; a
 // grouping with more raises ESP_STATUS_TILE_LIST (its grouped launches would miss tiles).
@@ -1064,7 +1064,7 @@ constexpr int TL_THREADS = 1024, TL_PER = 32;           // pairs a thread at mos
 
 __global__ __launch_bounds__(TL_THREADS) void tile_list_kernel(const int* __restrict__ ucount,
                                                               const int* __restrict__ members, int maxu, int maxm,
-                                                              int mt, int* __restrict__ tiles, int cap) {
+                                                              int mt, int rows, int* __restrict__ tiles, int cap) {
     __shared__ int wave_tot[TL_THREADS / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // the count and the first eight pairs' first members in flight together: every slot of the member table lies
@@ -1081,7 +1081,7 @@ __global__ __launch_bounds__(TL_THREADS) void tile_list_kernel(const int* __rest
             v[i] = -1;
             if (i0 + i < per && q < maxu * mt) {
                 const int u = q / mt, t = q - u * mt;
-                v[i] = members[(size_t)u * maxm + t * 32];
+                v[i] = members[(size_t)u * maxm + t * rows];
             }
         }
         if (pairs < 0) {
@@ -1674,6 +1674,13 @@ using namespace esp;
 
 static unsigned units_grid(long units, int per_block) { return (unsigned)((units + per_block - 1) / per_block); }
 
+// Whether a grouping runs as a workgroup an id (group_wide_kernel): past one workgroup's shared memory, and past 32 rows,
+// where one workgroup has no row bitmasks and each thread scans every pick for its experts (96 rows of 9 picks over 257
+// ids: ~160 us against 12)
+static bool wide_grouping(int64_t R, int64_t slots, int64_t maxm) {
+    return R * slots > MAX_PICKS || (R > 32 && maxm <= GW_MAX_M);
+}
+
 extern "C" int esp_group(const int32_t* pick, int32_t* uids, int64_t maxu, int32_t* ucount, int32_t* members,
                          int64_t maxm, int64_t R, int64_t slots, int64_t E, void* stream) {
     ESP_REQUIRE(pick && uids && ucount && members, "group: null pointer");
@@ -1682,7 +1689,7 @@ extern "C" int esp_group(const int32_t* pick, int32_t* uids, int64_t maxu, int32
     ESP_REQUIRE(R >= 1 && R * slots <= (int64_t(1) << 24), "grouping window too large");
     ESP_REQUIRE(maxu >= (R * slots < E ? R * slots : E), "uids too small");
     ESP_REQUIRE(maxm >= 1, "members too small");
-    if (R * slots > MAX_PICKS) {                     // past one workgroup's shared memory: a workgroup an id
+    if (wide_grouping(R, slots, maxm)) {
         ESP_REQUIRE(maxm <= GW_MAX_M, "group: at most 16384 members an expert");
         group_wide_kernel<<<(unsigned)E, GW, (size_t)maxm * 4, (hipStream_t)stream>>>(
             pick, (int)(R * slots), (int)slots, (int)E, (int)maxm, uids, ucount, members);
@@ -1854,7 +1861,7 @@ extern "C" int esp_group_shared(const int32_t* pick_in, const float* wts_in, con
     ESP_REQUIRE(!has || (H % 256 == 0 && x_stride % 4 == 0), "group_shared: H must be a multiple of 256");
     ESP_REQUIRE(maxu >= (R * slots < E ? R * slots : E), "uids too small");
     ESP_REQUIRE(maxm >= 1, "members too small");
-    if (R * slots > MAX_PICKS) {                     // past one workgroup's shared memory: the tables, then the grouping
+    if (wide_grouping(R, slots, maxm)) {             // the tables, then the grouping
         ESP_REQUIRE(maxm <= GW_MAX_M, "group_shared: at most 16384 members an expert");
         hipStream_t st = (hipStream_t)stream;
         shared_slots_kernel<<<(unsigned)((R + 3) / 4), 256, 0, st>>>(
@@ -1893,8 +1900,8 @@ extern "C" int esp_rot_in(const void* x, int x_dtype, int64_t x_stride, const in
 
 // the largest number of non-empty member tiles a grouping of P picks over nexp_max expert slots can have: the sum
 // over experts of ceil(members / 32) is at most P / 32 + the experts used
-static int64_t tile_list_cap(int64_t nexp_max, int64_t maxm, int64_t P) {
-    const int64_t mt = (maxm + 31) / 32, bound = (P + 31) / 32 + nexp_max;
+static int64_t tile_list_cap(int64_t nexp_max, int64_t maxm, int64_t P, int64_t rows = 32) {
+    const int64_t mt = (maxm + rows - 1) / rows, bound = (P + rows - 1) / rows + nexp_max;
     return nexp_max * mt < bound ? nexp_max * mt : bound;
 }
 
@@ -1975,17 +1982,24 @@ extern "C" int esp_grouped(const void* X0, const void* X1, const int64_t* TP0, c
                         N, P, SK, slots, warps, lo, hi, nullptr, stream);
 }
 
-extern "C" int esp_tile_list(const int32_t* ucount, const int32_t* members, int64_t nexp_max, int64_t maxm, int64_t P,
-                             int32_t* tiles, int64_t tiles_numel, void* stream) {
+extern "C" int esp_tile_list_rows(const int32_t* ucount, const int32_t* members, int64_t nexp_max, int64_t maxm,
+                                  int64_t P, int64_t rows, int32_t* tiles, int64_t tiles_numel, void* stream) {
     ESP_REQUIRE(ucount && members && tiles, "tile_list: null pointer");
     ESP_REQUIRE(nexp_max >= 1 && nexp_max < 65536 && maxm >= 1 && maxm <= 65536 && P >= 1,
                 "tile_list: 1 to 65535 expert slots, 1 to 65536 members a row, P >= 1");
-    const int64_t mt = (maxm + 31) / 32, cap = tile_list_cap(nexp_max, maxm, P);
+    ESP_REQUIRE(rows == 32 || rows == 64, "tile_list: tiles of 32 or 64 members");
+    const int64_t mt = (maxm + rows - 1) / rows, cap = tile_list_cap(nexp_max, maxm, P, rows);
     ESP_REQUIRE(nexp_max * mt <= (int64_t)TL_THREADS * TL_PER, "tile_list: at most 32768 (expert, member tile) pairs");
-    ESP_REQUIRE(tiles_numel >= 1 + cap, "tile_list: tiles needs 1 + min(E * ceil(maxm / 32), ceil(P / 32) + E) ints");
+    ESP_REQUIRE(tiles_numel >= 1 + cap,
+                "tile_list: tiles needs 1 + min(E * ceil(maxm / rows), ceil(P / rows) + E) ints (rows a tile)");
     tile_list_kernel<<<1, TL_THREADS, 0, (hipStream_t)stream>>>(ucount, members, (int)nexp_max, (int)maxm, (int)mt,
-                                                                tiles, (int)cap);
+                                                                (int)rows, tiles, (int)cap);
     return esp_host::launch_check("tile_list");
+}
+
+extern "C" int esp_tile_list(const int32_t* ucount, const int32_t* members, int64_t nexp_max, int64_t maxm, int64_t P,
+                             int32_t* tiles, int64_t tiles_numel, void* stream) {
+    return esp_tile_list_rows(ucount, members, nexp_max, maxm, P, 32, tiles, tiles_numel, stream);
 }
 
 extern "C" int esp_grouped_list(const void* X0, const void* X1, const int64_t* TP0, const int64_t* TP1,
@@ -2294,6 +2308,7 @@ extern "C" int esp_status(int32_t* status, int clear, void* stream) {
     if (esp_host::dense_status(clear, st, status)) return ESP_ERR_HIP;
     if (esp_host::tile_status(clear, st, status)) return ESP_ERR_HIP;
     if (esp_host::dense_own_status(clear, st, status)) return ESP_ERR_HIP;
+    if (esp_host::moe_prompt_status(clear, st, status)) return ESP_ERR_HIP;
     *status |= v;
     if (clear && v) {
         const int zero = 0;

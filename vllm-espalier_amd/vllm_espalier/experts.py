@@ -49,8 +49,7 @@ FUSED_ROWS = 4
 # (esp_moe_chain: the down programs decode their weights while gate/up runs; the same bits); ESPALIER_MOE_CHAIN=0 off
 CHAIN = env("ESPALIER_MOE_CHAIN", "1") != "0"
 CHAIN_ROWS = 4
-PREFILL_WAVES = 4          # waves a workgroup of the whole-prompt (prefill) grouped launches
-PREFILL_SK_GU = 1          # K splits of the whole-prompt gate/up launch
+PREFILL_WAVES = 4          # waves a workgroup of the whole-prompt grouped launches
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 
@@ -262,6 +261,16 @@ class Scratch:
         # the logits of esp_route_group_own and esp_route_group_rmsnorm (the shared gate's after each row's E): all-ones
         # between uses
         self.logits_n = torch.full((rows * (E + 1),), -1, dtype=i32, device=device).view(f32)
+        self.prompt: PrefillScratch | None = None        # windows' whole-prompt buffers, grown to the longest prompt
+        self.kept: list = []                             # outgrown ones that a captured graph may write to
+
+    def prompt_scratch(self, L: Layer, rows: int) -> PrefillScratch:
+        """The PrefillScratch of prompts of up to `rows` tokens that belongs to this scratch."""
+        if self.prompt is None or self.prompt.rows < rows:
+            if self.prompt is not None and self.prompt.captured:
+                self.kept.append(self.prompt)
+            self.prompt = PrefillScratch(L.E, L.D, L.I, rows, self.slots, self.z.device)
+        return self.prompt.handed_out()
 
     def window(self, R: int):
         """(ids, members [maxu, R]) views for a window of R tokens."""
@@ -390,18 +399,44 @@ def routed2(x: torch.Tensor, pick: torch.Tensor | None, wts: torch.Tensor | None
     return out, shared_out
 
 
+WINDOWS_PROMPT_ROWS = 2048     # tokens of one whole-prompt pass of windows (bounds its scratch)
+
+
+def _listed_rows(L: Layer) -> int:
+    """Tokens whose (expert, 32-token tile) pairs a tile list holds."""
+    return max(TILE_LIST_PAIRS // L.E, 1) * 32
+
+
+def _whole_prompt(x: torch.Tensor, L: Layer, gate: torch.Tensor | None) -> bool:
+    """Whether windows runs x's tokens as whole-prompt passes: past one window, with the rows as route_rows reads them
+    (16-byte aligned; the window launches take 8)."""
+    aligned = gate is None or (x.stride(0) % 8 == 0 and
+                               all(t is None or t.data_ptr() % 16 == 0 for t in (x, gate, L.gate_w)))
+    return x.stride(-1) == 1 and aligned and L.D % 128 == 0 and L.I % 128 == 0
+
+
 def windows(x: torch.Tensor, pick: torch.Tensor | None, wts: torch.Tensor | None, L: Layer, s: Scratch,
             k: int | None = None, gate: torch.Tensor | None = None):
-    """routed2 over consecutive windows of s.rows tokens (prefill), each exactly as in decode; with gate (and
-    pick=None), route() first in each window. Returns (routed sum, shared output or None)."""
+    """routed2 over any number of tokens (prefill), each exactly as in decode; with gate (and pick=None), route() first.
+    More than s.rows tokens run as whole-prompt passes (experts.prefill's launches with the window launches' K splits, so
+    their bits: each picked expert decoded once for up to 64 of its tokens instead of once a window), or as consecutive
+    windows of s.rows tokens. Returns (routed sum, shared output or None)."""
     out = torch.empty_like(x)
     shared_out = torch.empty_like(x) if L.shared_id >= 0 else None
-    for r0 in range(0, x.shape[0], s.rows):
-        rows = slice(r0, r0 + s.rows)
+    whole = x.shape[0] > s.rows and (pick is not None or gate is not None) and _whole_prompt(x, L, gate)
+    step = min(WINDOWS_PROMPT_ROWS, _listed_rows(L)) if whole else s.rows
+    for r0 in range(0, x.shape[0], step):
+        rows = slice(r0, r0 + step)
+        args = x[rows], None if pick is None else pick[rows], None if wts is None else wts[rows], L
+        outs = out[rows], None if shared_out is None else shared_out[rows]
+        if whole:
+            kk = k if pick is None else pick.shape[1]
+            ps = s.prompt_scratch(L, min(x.shape[0], step))
+            _prefill(*args, ps, kk, gate, *outs, s.cfg_gu[2], s.cfg_d[2])
+            continue
         if gate is not None:
             route(x[rows], gate, k, L, s)
-        routed2(x[rows], None if pick is None else pick[rows], None if wts is None else wts[rows], L, s,
-                out=out[rows], out_shared=None if shared_out is None else shared_out[rows], k=k)
+        routed2(*args, s, out=outs[0], out_shared=outs[1], k=k)
     return out, shared_out
 
 
@@ -412,12 +447,13 @@ class PrefillScratch:
 
     def __init__(self, E: int, D: int, I: int, rows: int, slots: int, device, window: int = 32):
         self.rows, self.slots, self.E, self.window = rows, slots, E, window
+        self.captured = False                            # handed out during a graph capture
         P = rows * slots
         maxu = min(P, E)
         f16, f32, i32 = torch.float16, torch.float32, torch.int32
         layout = {
             "xg": ((P, D), f16, 0), "xu": ((P, D), f16, 0), "xd": ((P, I), f16, 0),
-            "z": ((P * max(2 * I * PREFILL_SK_GU, D),), f32, 0),     # the gate/up splits' partials, or down's sums
+            "z": ((P * max(2 * I, D),), f32, 0),                     # the gate and up sums, or down's
             "pick": ((P,), i32, 0), "wts": ((P,), f32, 0),
             "ids": ((maxu,), i32, 0), "count": ((1,), i32, 0), "members": ((maxu * rows,), i32, -1),
             "tiles": ((1 + tile_list_cap(maxu, rows, P),), i32, 0),
@@ -426,18 +462,32 @@ class PrefillScratch:
         for name, (shape, dtype, fill) in layout.items():
             setattr(self, name, torch.full(shape, fill, dtype=dtype, device=device))
 
+    def handed_out(self) -> PrefillScratch:
+        self.captured |= torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
+        return self
+
     def grouping(self, T: int):
         maxu = min(T * self.slots, self.E)
         return self.ids[:maxu], self.members[:maxu * T].view(maxu, T)
 
 
 _PREFILL: dict = {}
+_PREFILL_KEPT: list = []     # outgrown prompt scratches that a captured graph may write to
 TILE_LIST_PAIRS = 32768      # esp_tile_list's limit on (expert slot, member tile) pairs
 
 
-def tile_list_cap(maxu: int, maxm: int, P: int) -> int:
-    """Entries esp_tile_list may write for a grouping of P picks over maxu expert slots, maxm members a row."""
-    return min(maxu * -(-maxm // 32), -(-P // 32) + maxu)
+def tile_list_cap(maxu: int, maxm: int, P: int, rows: int = 32) -> int:
+    """Entries esp_tile_list may write for a grouping of P picks over maxu expert slots, maxm members a row, in tiles of
+    `rows` members."""
+    return min(maxu * -(-maxm // rows), -(-P // rows) + maxu)
+
+
+def tile_rows(T: int, k: int, E: int) -> int:
+    """Members a tile of the whole-prompt expert launches (32 or 64; the same bits): 64 once a routed expert has more than
+    22 members on average, when enough experts pass 32 that decoding them once pays for the three waves a SIMD that
+    four row groups leave (a 256-expert layer, MI355X: 512 / 640 / 768 / 1024 / 1531 tokens 290 / 316 / 345 / 443 / 601 us
+    in tiles of 32, 296 / 324 / 337 / 385 / 458 us in tiles of 64)."""
+    return 64 if T * k > 22 * E else 32
 
 
 def prefill_scratch(layer: Layer, rows: int, slots: int, device) -> PrefillScratch:
@@ -445,8 +495,10 @@ def prefill_scratch(layer: Layer, rows: int, slots: int, device) -> PrefillScrat
     key = (layer.E, layer.D, layer.I, slots, str(device))
     found = _PREFILL.get(key)
     if found is None or found.rows < rows:
+        if found is not None and found.captured:
+            _PREFILL_KEPT.append(found)
         found = _PREFILL[key] = PrefillScratch(layer.E, layer.D, layer.I, rows, slots, device)
-    return found
+    return found.handed_out()
 
 
 PREFILL_MAX_ROWS = 16384    # tokens one whole-prompt grouping takes (the wide grouping's members an expert)
@@ -460,21 +512,23 @@ def prefill(x: torch.Tensor, pick: torch.Tensor | None, wts: torch.Tensor | None
     over that grouping with one K split, so each picked expert's weights are decoded once for all its member rows
     (in tiles of 32) instead of once a 32-token window. Returns (routed sum, shared output or None), [T, D] in x's
     dtype; a token's output depends on its own picks and rows only (the K split is fixed), not on the other tokens.
-    A prompt of more than PREFILL_MAX_ROWS tokens runs as consecutive chunks of that many (the same bits a row)."""
+    A prompt of more than PREFILL_MAX_ROWS tokens, or of more (expert, 32-token tile) pairs than a tile list holds, runs as
+    consecutive chunks (the same bits a row)."""
     T = x.shape[0]
-    if T <= PREFILL_MAX_ROWS:
+    step = min(PREFILL_MAX_ROWS, _listed_rows(L))
+    if T <= step:
         return _prefill(x, pick, wts, L, s, k, gate, out, out_shared)
     out = torch.empty((T, L.D), dtype=x.dtype, device=x.device) if out is None else out
     if L.shared_id >= 0 and out_shared is None:
         out_shared = torch.empty((T, L.D), dtype=x.dtype, device=x.device)
-    for r0 in range(0, T, PREFILL_MAX_ROWS):
-        rows = slice(r0, r0 + PREFILL_MAX_ROWS)
+    for r0 in range(0, T, step):
+        rows = slice(r0, r0 + step)
         _prefill(x[rows], None if pick is None else pick[rows], None if wts is None else wts[rows], L, s, k, gate,
                  out[rows], None if out_shared is None else out_shared[rows])
     return out, (out_shared if L.shared_id >= 0 else None)
 
 
-def _prefill(x, pick, wts, L: Layer, s: PrefillScratch, k: int, gate, out, out_shared):
+def _prefill(x, pick, wts, L: Layer, s: PrefillScratch, k: int, gate, out, out_shared, sk_gu: int = 1, sk_d: int = 1):
     e = ext()
     T = x.shape[0]
     has_shared = L.shared_id >= 0
@@ -493,23 +547,16 @@ def _prefill(x, pick, wts, L: Layer, s: PrefillScratch, k: int, gate, out, out_s
         e.group_shared(pick, wts, x, x.stride(0), L.gate_w, L.shared_id, pick_p, wts_p, ids, s.count, members, T, k,
                        L.E)
     e.rot_in(x, x.stride(0), pick_p, L.suh_g, L.suh_u, s.xg, s.xu, T, L.D, slots, L.E)
-    sk = PREFILL_SK_GU
     t, b, c = L.ptr[2], L.k2[2], L.cb[2]
-    # the grouped launches over the grouping's non-empty (expert, member tile) pairs only: a grid of every expert slot
-    # times every member tile is mostly empty workgroups (the same programs either way, the same bits)
-    if ids.numel() * -(-T // 32) <= TILE_LIST_PAIRS:
-        e.tile_list(s.count, members, ids.numel(), P, s.tiles)
-        e.grouped_list(s.xg, s.xu, L.ptr[0], L.ptr[1], L.k2[0], L.k2[1], L.cb[0], L.cb[1], ids, s.count, members,
-                       s.tiles, s.z, 2, L.D, L.I, P, sk, slots, PREFILL_WAVES, *L.k2_gu)
-        e.gateup_epilogue(s.z, pick_p, L.svh_g, L.svh_u, L.suh_d, s.xd, T, P, L.I, sk, slots, L.E, math.inf, ACT_F32)
-        e.grouped_list(s.xd, s.xd, t, t, b, b, c, c, ids, s.count, members, s.tiles, s.z, 1, L.I, L.D, P, 1, slots,
-                       PREFILL_WAVES, *L.k2_d)
-    else:
-        e.grouped(s.xg, s.xu, L.ptr[0], L.ptr[1], L.k2[0], L.k2[1], L.cb[0], L.cb[1], ids, s.count, members, s.z, 2,
-                  L.D, L.I, P, sk, slots, 8, PREFILL_WAVES, 2, *L.k2_gu)
-        e.gateup_epilogue(s.z, pick_p, L.svh_g, L.svh_u, L.suh_d, s.xd, T, P, L.I, sk, slots, L.E, math.inf, ACT_F32)
-        e.grouped(s.xd, s.xd, t, t, b, b, c, c, ids, s.count, members, s.z, 1, L.I, L.D, P, 1, slots, 8,
-                  PREFILL_WAVES, 2, *L.k2_d)
+    # over the grouping's non-empty (expert, member tile) pairs only: a grid of every expert slot times every member tile
+    # is mostly empty workgroups
+    tr = tile_rows(T, k, L.E - has_shared)
+    e.tile_list(s.count, members, ids.numel(), P, s.tiles, tr)
+    e.grouped_prompt(s.xg, s.xu, L.ptr[0], L.ptr[1], L.k2[0], L.k2[1], L.cb[0], L.cb[1], ids, s.count, members, s.tiles,
+                     tr, s.z, 2, L.D, L.I, P, sk_gu, slots, *L.k2_gu)
+    e.gateup_epilogue(s.z, pick_p, L.svh_g, L.svh_u, L.suh_d, s.xd, T, P, L.I, 1, slots, L.E, math.inf, ACT_F32)
+    e.grouped_prompt(s.xd, s.xd, t, t, b, b, c, c, ids, s.count, members, s.tiles, tr, s.z, 1, L.I, L.D, P, sk_d, slots,
+                     *L.k2_d)
     out = torch.empty((T, L.D), dtype=x.dtype, device=x.device) if out is None else out
     if has_shared and out_shared is None:
         out_shared = torch.empty((T, L.D), dtype=x.dtype, device=x.device)
