@@ -101,3 +101,15 @@ def test_prompt_graph_replay(dev):
         torch.cuda.synchronize()
         assert torch.equal(y, want), i
         torch.randn((64, 64), device=dev).sum()                # eager work between replays
+
+
+def test_tile_mode_few_rows_of_a_wide_layer(dev):
+    """A layer with one K split and two k slots (an LM head's plan): up to 32 rows of the tile mode are decode launches,
+    with the bits of the same rows in a longer prompt."""
+    gen = torch.Generator().manual_seed(3)
+    d = D.Dense([WL.matrix(256, 128 * 260, 2, "mcg", gen, dev)])
+    assert d._tile_is_window(32, d.launches[0]) and not d._tile_is_window(33, d.launches[0])
+    x = _rows(100, d.K, torch.bfloat16, dev, 2)
+    y = d.forward_tile(x)
+    for T in (1, 7, 32):
+        assert torch.equal(d.forward_tile(x[:T]), y[:T]), T

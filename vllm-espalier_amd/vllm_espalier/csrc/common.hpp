@@ -189,6 +189,109 @@ __device__ __forceinline__ uint2 rot128(const void* x, int x_dtype, size_t xi, c
     return rot128_apply(rot128_load(x, x_dtype, xi, suh, lane32), x_dtype, lane32);
 }
 
+// The same transform with 16 values a lane, 8 lanes (l8 = lane & 7) a 128-block: 16 / R runs of R consecutive elements,
+// v[i] element run16<R>(l8, i). Strides below R and from 8 R on are in a lane's registers, the three between across lanes;
+// every butterfly and its place in the order are fwht128's, so the bits are too, in half the instructions an element
+// (three exchanges of 16 values against five of 4 over four times the lanes). For work bound by issue; fwht128 spreads a
+// block over a whole half-wave, for work bound by latency (the dense launches' rotation of 32 rows: 526 -> 537 us over 48
+// launches with this form). R = 4 moves fp32 rows 16 bytes a lane, 128 a block, R = 16 suits a prompt's fragments.
+template <int R>
+__device__ __forceinline__ int run16(int l8, int i) {
+    return i / R * (8 * R) + R * l8 + i % R;
+}
+
+template <int S>
+__device__ __forceinline__ void fwht_regs16(float (&v)[16]) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+        if (!(i & S)) {
+            const float p = v[i], o = v[i + S];
+            v[i] = p + o;
+            v[i + S] = p - o;
+        }
+}
+
+template <int M>
+__device__ __forceinline__ void fwht_lanes16(float (&v)[16], int lane) {
+    const uint32_t neg = lane & M ? 0x80000000u : 0u;                  // the upper lane takes o - v
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+        v[i] = xor_lane32<M>(v[i]) + __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[i]) ^ neg);
+}
+
+template <int R>
+__device__ __forceinline__ void fwht128_16(float (&v)[16], int lane) {
+    static_assert(R == 4 || R == 16, "run length");
+    fwht_regs16<1>(v);
+    fwht_regs16<2>(v);
+    if constexpr (R == 16) {
+        fwht_regs16<4>(v);
+        fwht_regs16<8>(v);
+    }
+    fwht_lanes16<1>(v, lane);
+    fwht_lanes16<2>(v, lane);
+    fwht_lanes16<4>(v, lane);
+    if constexpr (R == 4) {
+        fwht_regs16<4>(v);
+        fwht_regs16<8>(v);
+    }
+}
+
+// a lane's 16 fp16 / bf16 bit patterns of the 128 at p, two a word (p 8-byte aligned; 16 with `wide`, used for R > 4)
+template <int R>
+__device__ __forceinline__ void load16_bits(const uint16_t* p, bool wide, int l8, uint32_t (&w)[8]) {
+    if (R > 4 && wide) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint4 a = *reinterpret_cast<const uint4*>(p + run16<R>(l8, 8 * i));
+            w[4 * i] = a.x; w[4 * i + 1] = a.y; w[4 * i + 2] = a.z; w[4 * i + 3] = a.w;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint2 a = *reinterpret_cast<const uint2*>(p + run16<R>(l8, 4 * i));
+            w[2 * i] = a.x;
+            w[2 * i + 1] = a.y;
+        }
+    }
+}
+
+__device__ __forceinline__ uint16_t half_of(const uint32_t (&w)[8], int i) { return (uint16_t)(w[i >> 1] >> (16 * (i & 1))); }
+
+// a lane's 16 of the 128 floats at p (16-byte aligned)
+template <int R>
+__device__ __forceinline__ void load16_f32(const float* p, int l8, float (&v)[16]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float4 t = *reinterpret_cast<const float4*>(p + run16<R>(l8, 4 * i));
+        v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
+    }
+}
+
+// rot128's fp16 H(x * suh) / sqrt(128) of the 128 elements of x from xi, with 16 a lane, as 8 packed words. wide: x + xi
+// and suh 16-byte aligned (8 otherwise; fp32 rows always 16).
+template <int R>
+__device__ __forceinline__ void rot128_16(const void* x, int x_dtype, size_t xi, const uint16_t* suh, bool wide, int lane,
+                                          uint32_t (&r)[8]) {
+    const int l8 = lane & 7;
+    float v[16];
+    uint32_t xw[8], sw[8];
+    load16_bits<R>(suh, wide, l8, sw);
+    if (x_dtype == F32) {
+        load16_f32<R>(static_cast<const float*>(x) + xi, l8, v);
+    } else {
+        load16_bits<R>(static_cast<const uint16_t*>(x) + xi, wide, l8, xw);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = x_dtype == BF16 ? bf2f(half_of(xw, i)) : h2f(half_of(xw, i));
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = __fmul_rn(v[i], h2f(half_of(sw, i)));
+    fwht128_16<R>(v, lane);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        r[i] = (uint32_t)f2h(v[2 * i] * HAD_SCALE) | ((uint32_t)f2h(v[2 * i + 1] * HAD_SCALE) << 16);
+}
+
 // ---- hand-off of partial results between workgroups ----
 // MI355X's eight XCDs each have their own L2, so an agent-scope release fence writes back the whole L2 (buffer_wbl2):
 // ~100 ns a fence, serialised per XCD, which at thousands of waves a launch costs more than the GEMM. Partials

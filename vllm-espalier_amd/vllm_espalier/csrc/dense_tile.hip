@@ -103,16 +103,13 @@ __device__ __forceinline__ void tile_all_arrived(int* counter, int* seen, int to
     __syncthreads();
 }
 
-// xh, a (matrix, row group, 128-chunk) a workgroup
 __global__ __launch_bounds__(256) void tile_rot_kernel(const void* __restrict__ x, int x_dtype, int x_stride, int T,
-                                                       int K, int n, const uint16_t* suh0, const uint16_t* suh1,
-                                                       const uint16_t* suh2, const uint16_t* suh3,
+                                                       int K, bool wide, unsigned units, const uint16_t* suh0,
+                                                       const uint16_t* suh1, const uint16_t* suh2, const uint16_t* suh3,
                                                        uint16_t* __restrict__ xh, int RG) {
-    __shared__ __align__(16) uint16_t frag[4 * TILE_FRAG];
-    int ch;
-    uint16_t* dst = tile_rot_unit(blockIdx.x, x, x_dtype, x_stride, T, K, suh0, suh1, suh2, suh3, xh, RG, frag, ch) +
-                    (size_t)ch * 4 * TILE_FRAG;              // the chunk's 4 KiB, one 16-byte store a thread
-    reinterpret_cast<uint4*>(dst)[threadIdx.x] = reinterpret_cast<const uint4*>(frag)[threadIdx.x];
+    const unsigned unit = blockIdx.x * ROT_UNITS + (threadIdx.x >> 3);
+    if (unit < units)
+        tile_rot_unit(unit, x, x_dtype, x_stride, T, K, wide, suh0, suh1, suh2, suh3, xh, RG, [](int st) { return st; });
 }
 
 // The finisher's rows of one half-wave (rows rbase, rbase + 16, ...): RPB rows at a time with the other splits'
@@ -560,10 +557,11 @@ extern "C" int esp_dense_tile(const void* x, int x_dtype, int64_t x_stride, int6
     const size_t red = (size_t)RED_BYTES + 16;                   // the sums, then the arrival flag
     const size_t smem = stage > red ? stage : red;
     hipStream_t st = (hipStream_t)stream;
-    const long units = (long)n_shards * RG * (K / 128);          // (matrix, row group, 128-chunk)
-    tile_rot_kernel<<<(unsigned)units, 256, 0, st>>>(x, x_dtype, (int)x_stride, (int)T, (int)K,
-                                                                 (int)n_shards, su[0], su[1], su[2], su[3],
-                                                                 static_cast<uint16_t*>(xh), (int)RG);
+    const long units = (long)n_shards * RG * (K / 128) * 16;     // (matrix, row, 128-chunk)
+    ESP_REQUIRE(units < (long)1 << 31, "dense_tile: too many rows for one launch");
+    tile_rot_kernel<<<(unsigned)((units + ROT_UNITS - 1) / ROT_UNITS), 256, 0, st>>>(
+        x, x_dtype, (int)x_stride, (int)T, (int)K, rot_wide(x, x_stride, su, (int)n_shards), (unsigned)units, su[0], su[1],
+        su[2], su[3], static_cast<uint16_t*>(xh), (int)RG);
     int rc = esp_host::launch_check("dense_tile rotation");
     if (rc) return rc;
     const dim3 grid((unsigned)nbt, (unsigned)SK, (unsigned)tiles);

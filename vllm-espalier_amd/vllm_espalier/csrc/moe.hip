@@ -975,82 +975,100 @@ __global__ __launch_bounds__(1024) void down_combine_kernel(const float* __restr
                                  blockIdx.y, part);
 }
 
-// down_combine for many rows (a prompt): one workgroup (8 32-lane halves) a (row, group of DCR_BLOCKS 128-blocks), the
-// row's picks and weights read once into shared memory for the group; a half-wave takes up to DCR_U (slot, block)
-// units of the group with all their loads in flight, then the fma chain in slot order over the group's columns.
-// Element for element the arithmetic of down_combine_unit (a workgroup a (row, 128-block)), which the few-row launches
-// keep.
-constexpr int DCR_BLOCKS = 4, DCR_U = 5, DCR_ROWS = 64;   // DCR_ROWS: rows from which esp_down_combine* use this form
+// down_combine for many rows (a prompt): 8 lanes a (row, 128-block), 16 columns a lane, a wave a workgroup. The row's
+// slots pass in order through the lane's registers, DCR_SLOTS of them with their loads in flight, so the routed fma chain
+// needs no shared memory; element for element the arithmetic of down_combine_unit, which the few-row launches keep.
+// Bound by the partials' bytes: 1531 tokens of 9 slots, D = 2048 (113 MB): 49 -> 25 us (4.5 TB/s) against the slots spread
+// over half-waves and the chain through shared memory; 391 tokens 16.6 -> 14.5 us. (The same layout for rot_in and
+// gateup_epilogue was slower there, 40 -> 47 and 20.8 -> 22.4 us at 1531 tokens: they wait for memory, not for issue.)
+constexpr int DCR_SLOTS = 3, DCR_ROWS = 64;            // DCR_ROWS: rows from which esp_down_combine* use this form
+
+// a lane's 16 of a row's 128 outputs (aligned: 16-bit rows 8 bytes, fp32 rows 16; else one by one)
+template <int OUT_DTYPE>
+__device__ __forceinline__ void store16_out(void* out, size_t at, const float (&v)[16], bool aligned, int l8) {
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) {
+        const size_t j = at + run16<4>(l8, i);
+        const float w[4] = {v[i], v[i + 1], v[i + 2], v[i + 3]};
+        if (aligned) {
+            store4(out, OUT_DTYPE, j, w);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if constexpr (OUT_DTYPE == F32) static_cast<float*>(out)[j + q] = w[q];
+                else static_cast<uint16_t*>(out)[j + q] = OUT_DTYPE == BF16 ? f2bf(w[q]) : f2h(w[q]);
+            }
+        }
+    }
+}
 
 template <int OUT_DTYPE>
-__global__ __launch_bounds__(256) void down_combine_rows_kernel(const float* __restrict__ Z,
-                                                                const int* __restrict__ pick,
-                                                                const uint16_t* __restrict__ svh_d,
-                                                                float* __restrict__ y, const float* __restrict__ wts,
-                                                                void* __restrict__ out, void* __restrict__ out_shared,
-                                                                int P, int D, int SK, int E, int slots, int n_routed) {
-    extern __shared__ float dcr_part[];                      // [slots][DCR_BLOCKS * 128]
-    __shared__ float wts_sh[32];
-    __shared__ int e_sh[32];
-    constexpr int GW = DCR_BLOCKS * 128;
-    const int r = blockIdx.x, l32 = threadIdx.x & 31, hw = threadIdx.x >> 5;
-    if ((int)threadIdx.x < slots) {
-        wts_sh[threadIdx.x] = wts[r * slots + threadIdx.x];
-        e_sh[threadIdx.x] = pick[r * slots + threadIdx.x];
-    }
-    __syncthreads();
-    const int nbt = D >> 7;
-    {
-        const int b0 = blockIdx.y * DCR_BLOCKS;
-        const int nbk = nbt - b0 < DCR_BLOCKS ? nbt - b0 : DCR_BLOCKS, units = slots * nbk;
-        for (int u0 = hw; u0 < units; u0 += 8 * DCR_U) {
-            float v[DCR_U][4], sv[DCR_U][4];
+__global__ __launch_bounds__(64) void down_combine_rows_kernel(const float* __restrict__ Z, const int* __restrict__ pick,
+                                                               const uint16_t* __restrict__ svh_d,
+                                                               float* __restrict__ y, const float* __restrict__ wts,
+                                                               void* __restrict__ out, void* __restrict__ out_shared,
+                                                               int rows, int P, int D, int SK, int E, int slots,
+                                                               int n_routed, bool aligned) {
+    const int lane = threadIdx.x, l8 = lane & 7, nb = D >> 7;
+    const long unit = (long)blockIdx.x * 8 + (lane >> 3);
+    if (unit >= (long)rows * nb) return;
+    const int r = (int)(unit / nb), n = (int)(unit % nb) * 128;
+    const size_t at = (size_t)r * D + n;
+    const int last = out_shared != nullptr && n_routed < slots ? n_routed + 1 : n_routed;
+    const int used = y != nullptr ? slots : last;          // the slots past them only store their outputs
+    float acc[16];
 #pragma unroll
-            for (int i = 0; i < DCR_U; ++i) {               // every unit's loads first
-                const int u = u0 + 8 * i;
-                if (u < units) {
-                    const int k = u / nbk, n = (b0 + u - k * nbk) * 128 + 4 * l32, e = e_sh[k];
-                    sum_splits4(Z + (size_t)(r * slots + k) * D + n, (size_t)P * D, SK, v[i]);
-                    if (e >= 0 && e < E) load4_f16(svh_d + (size_t)e * D + n, sv[i]);
-                }
-            }
+    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+    for (int k0 = 0; k0 < used; k0 += DCR_SLOTS) {
+        float v[DCR_SLOTS][16], w[DCR_SLOTS];
+        uint32_t sv[DCR_SLOTS][8];
+        int e[DCR_SLOTS];
 #pragma unroll
-            for (int i = 0; i < DCR_U; ++i) {
-                const int u = u0 + 8 * i;
-                if (u < units) {                            // uniform over the half-wave
-                    const int k = u / nbk, bl = u - k * nbk, n = (b0 + bl) * 128 + 4 * l32, e = e_sh[k];
-                    const size_t pi = (size_t)(r * slots + k) * D + n;
-                    float o[4];
-                    if (e >= 0 && e < E) {
-                        fwht128(v[i], l32);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) o[j] = v[i][j] * HAD_SCALE * sv[i][j];
-                        if (y != nullptr) *reinterpret_cast<float4*>(y + pi) = make_float4(o[0], o[1], o[2], o[3]);
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) o[j] = y != nullptr ? y[pi + j] : 0.f;   // reuses y's row
-                    }
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) dcr_part[k * GW + bl * 128 + 4 * l32 + j] = o[j];
-                }
-            }
+        for (int q = 0; q < DCR_SLOTS; ++q) {
+            const int k = k0 + q < used ? k0 + q : used - 1, p = r * slots + k;       // past the last: read, not used
+            e[q] = pick[p];
+            w[q] = wts[p];
+            load16_f32<4>(Z + (size_t)p * D + n, l8, v[q]);
         }
-        __syncthreads();
-        for (int c = threadIdx.x; c < nbk * 128; c += 256) {
-            const size_t at = (size_t)r * D + b0 * 128 + c;
-            float acc = 0.f;
-            for (int q = 0; q < n_routed; ++q) acc = fmaf(wts_sh[q], dcr_part[q * GW + c], acc);
-            if constexpr (OUT_DTYPE == F32) static_cast<float*>(out)[at] = acc;
-            else if constexpr (OUT_DTYPE == BF16) static_cast<uint16_t*>(out)[at] = f2bf(acc);
-            else static_cast<uint16_t*>(out)[at] = f2h(acc);
-            if (out_shared != nullptr && n_routed < slots) {
-                const float sv1 = wts_sh[n_routed] * dcr_part[n_routed * GW + c];
-                if constexpr (OUT_DTYPE == F32) static_cast<float*>(out_shared)[at] = sv1;
-                else if constexpr (OUT_DTYPE == BF16) static_cast<uint16_t*>(out_shared)[at] = f2bf(sv1);
-                else static_cast<uint16_t*>(out_shared)[at] = f2h(sv1);
+#pragma unroll
+        for (int q = 0; q < DCR_SLOTS; ++q)
+            load16_bits<4>(svh_d + (size_t)(e[q] >= 0 && e[q] < E ? e[q] : 0) * D + n, false, l8, sv[q]);
+#pragma unroll
+        for (int q = 0; q < DCR_SLOTS; ++q) {
+            const int k = k0 + q;
+            if (k >= used) break;
+            const size_t pi = (size_t)(r * slots + k) * D + n;
+            for (int s = 1; s < SK; ++s) {
+                float u[16];
+                load16_f32<4>(Z + (size_t)s * P * D + pi, l8, u);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[q][i] += u[i];
+            }
+            const bool valid = e[q] >= 0 && e[q] < E;       // the same in the unit's 8 lanes
+            if (valid) {
+                fwht128_16<4>(v[q], lane);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[q][i] = v[q][i] * HAD_SCALE * h2f(half_of(sv[q], i));
+                if (y != nullptr)
+#pragma unroll
+                    for (int i = 0; i < 16; i += 4)
+                        *reinterpret_cast<float4*>(y + pi + run16<4>(l8, i)) =
+                            make_float4(v[q][i], v[q][i + 1], v[q][i + 2], v[q][i + 3]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[q][i] = y != nullptr ? y[pi + run16<4>(l8, i)] : 0.f;   // reuses y's row
+            }
+            if (k < n_routed) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[i] = fmaf(w[q], v[q][i], acc[i]);
+            } else if (k == n_routed && out_shared != nullptr) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[q][i] = w[q] * v[q][i];
+                store16_out<OUT_DTYPE>(out_shared, at, v[q], aligned, l8);
             }
         }
     }
+    store16_out<OUT_DTYPE>(out, at, acc, aligned, l8);
 }
 
 // ------------------------------------------------------------------------------------------------------------------
@@ -2254,19 +2272,22 @@ static int down_combine_any(const float* Z, const int32_t* pick, const void* svh
     if (rows <= 0) return esp_host::ok();
     hipStream_t s = (hipStream_t)stream;
     auto svh = static_cast<const uint16_t*>(svh_d);
-    if (rows >= DCR_ROWS) {                                 // a workgroup a (row, 4 128-blocks)
-        ESP_REQUIRE(rows < (int64_t(1) << 31), "down_combine: at most 2^31 - 1 rows");
-        const size_t smem = (size_t)slots * DCR_BLOCKS * 128 * 4;
-        const dim3 g((unsigned)rows, (unsigned)((D / 128 + DCR_BLOCKS - 1) / DCR_BLOCKS));
+    // 8 lanes a (row, 128-block); they read Z and y 16 bytes at a time
+    if (rows >= DCR_ROWS && (((uintptr_t)Z | (uintptr_t)y) & 15) == 0 && ((uintptr_t)svh_d & 7) == 0) {
+        const long units = rows * (D / 128);
+        ESP_REQUIRE(units < (long)1 << 33 && rows < (int64_t(1) << 31), "down_combine: at most 2^31 - 1 rows");
+        const bool aligned = (((uintptr_t)out | (uintptr_t)out_shared) & 15) == 0;
+        const unsigned g = units_grid(units, 8);
+#define ESP_DCR(T)                                                                                                  \
+    down_combine_rows_kernel<T><<<g, 64, 0, s>>>(Z, pick, svh, y, wts, out, out_shared, (int)rows, (int)P, (int)D, \
+                                                 (int)SK, (int)E, (int)slots, (int)n_routed, aligned)
         if (out_dtype == ESP_BF16)
-            down_combine_rows_kernel<BF16><<<g, 256, smem, s>>>(Z, pick, svh, y, wts, out, out_shared, (int)P, (int)D,
-                                                                (int)SK, (int)E, (int)slots, (int)n_routed);
+            ESP_DCR(BF16);
         else if (out_dtype == ESP_F16)
-            down_combine_rows_kernel<F16><<<g, 256, smem, s>>>(Z, pick, svh, y, wts, out, out_shared, (int)P, (int)D,
-                                                               (int)SK, (int)E, (int)slots, (int)n_routed);
+            ESP_DCR(F16);
         else
-            down_combine_rows_kernel<F32><<<g, 256, smem, s>>>(Z, pick, svh, y, wts, out, out_shared, (int)P, (int)D,
-                                                               (int)SK, (int)E, (int)slots, (int)n_routed);
+            ESP_DCR(F32);
+#undef ESP_DCR
         return esp_host::launch_check("down_combine");
     }
     dim3 grid((unsigned)rows, (unsigned)(D / 128));

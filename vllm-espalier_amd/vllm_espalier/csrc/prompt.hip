@@ -49,7 +49,8 @@ struct PrepArgs {
     int rows, K, RG, NBT;
     uint16_t* xh;
     uint16_t* wf;
-    unsigned rot_units;                       // workgroups that rotate; the others decode
+    bool wide;                                // rot128_16's
+    unsigned rot_units, rot_wgs;              // rows to rotate, and the workgroups that do; the others decode
 };
 
 constexpr int PREP_WAVES = 4;                 // waves of a decoding workgroup, a 32-k step each
@@ -58,20 +59,18 @@ constexpr int PREP_WAVES = 4;                 // waves of a decoding workgroup, 
 // lane decodes its B operand of the 8 n tiles and stores it as 16 bytes, a wave a KiB.
 template <int CB, int K2>
 __global__ __launch_bounds__(256) void prompt_prep_kernel(PrepArgs a) {
-    __shared__ __align__(16) uint32_t smem[K2 * PREP_WAVES * 64 > 4 * TILE_FRAG / 2 ? K2 * PREP_WAVES * 64 : 4 * TILE_FRAG / 2];
-    if (blockIdx.x < a.rot_units) {
-        int ch;
-        uint16_t* frag = reinterpret_cast<uint16_t*>(smem);
-        uint16_t* rows = tile_rot_unit(blockIdx.x, a.x, a.x_dtype, a.x_stride, a.rows, a.K, a.suh[0], a.suh[1], a.suh[2],
-                                       a.suh[3], a.xh, a.RG, frag, ch);
-        uint16_t* dst = rows + (size_t)a.order.place(ch * 4 + (threadIdx.x >> 6)) * TILE_FRAG;
-        reinterpret_cast<uint4*>(dst)[threadIdx.x & 63] = reinterpret_cast<const uint4*>(frag)[threadIdx.x];
+    __shared__ __align__(16) uint32_t smem[K2 * PREP_WAVES * 64];
+    if (blockIdx.x < a.rot_wgs) {
+        const unsigned unit = blockIdx.x * ROT_UNITS + (threadIdx.x >> 3);
+        if (unit < a.rot_units)
+            tile_rot_unit(unit, a.x, a.x_dtype, a.x_stride, a.rows, a.K, a.wide, a.suh[0], a.suh[1], a.suh[2], a.suh[3],
+                          a.xh, a.RG, [&](int st) { return a.order.place(st); });
         return;
     }
     constexpr int TW = 4 * K2, ROW = 8 * TW;             // words of a tile, of a k tile of the block
     const int steps = a.K >> 5, groups = steps / PREP_WAVES;                  // K % 128 == 0
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, G = lane >> 4;
-    const int unit = (int)(blockIdx.x - a.rot_units), nbg = unit / groups, step = (unit - nbg * groups) * PREP_WAVES + wave;
+    const int unit = (int)(blockIdx.x - a.rot_wgs), nbg = unit / groups, step = (unit - nbg * groups) * PREP_WAVES + wave;
     const uint32_t* T = a.T[0];
     int nb0 = a.nb0[0], nb = a.nb[0];
 #pragma unroll
@@ -295,21 +294,13 @@ __global__ __launch_bounds__(PG_WAVES * 64, 3) void prompt_gemm_kernel(PromptArg
         }
     }
 
-    // the tile's sums through shared memory: 8 lanes a row, 16 columns a lane, for the output transform (the butterflies
-    // of fwht128 in its order: strides 1 to 8 in a lane's registers, 16 to 64 across lanes)
+    // the tile's sums through shared memory: 8 lanes a row, 16 columns a lane, for the output transform
     const int cb_local = nbg - nb0, l8 = lane & 7;
     const uint2* sp = reinterpret_cast<const uint2*>(svh + cb_local * 128 + 16 * l8);          // 8-byte aligned
     const uint2 s0 = sp[0], s1 = sp[1], s2 = sp[2], s3 = sp[3];
     const uint32_t sw[8] = {s0.x, s0.y, s1.x, s1.y, s2.x, s2.y, s3.x, s3.y};
     float* red = reinterpret_cast<float*>(smem);
     const int ycol = col0 + cb_local * 128 + 16 * l8;
-    auto butterfly = [&](float (&v)[16], auto m) __attribute__((always_inline)) {
-        constexpr int M = decltype(m)::value;
-        const uint32_t neg = lane & M ? 0x80000000u : 0u;              // the upper lane takes o - v
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            v[i] = xor_lane32<M>(v[i]) + __uint_as_float(__float_as_uint(v[i]) ^ neg);
-    };
     wait_vm_lgkm0<0>();                                                // every copy landed, every fragment read
     __syncthreads();
 #pragma unroll
@@ -329,18 +320,7 @@ __global__ __launch_bounds__(PG_WAVES * 64, 3) void prompt_gemm_kernel(PromptArg
             const float4 t = *reinterpret_cast<const float4*>(red + r * RED_STRIDE + 16 * l8 + 4 * i);
             v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
         }
-#pragma unroll
-        for (int st = 1; st < 16; st *= 2)
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-                if (!(i & st)) {
-                    const float p = v[i], o = v[i + st];
-                    v[i] = p + o;
-                    v[i + st] = p - o;
-                }
-        butterfly(v, std::integral_constant<int, 1>{});
-        butterfly(v, std::integral_constant<int, 2>{});
-        butterfly(v, std::integral_constant<int, 4>{});
+        fwht128_16<16>(v, lane);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             v[i] *= a.scale;
@@ -404,7 +384,7 @@ extern "C" int esp_dense_prompt(const void* x, int x_dtype, int64_t x_stride, in
     const int64_t RG = (T + 15) / 16;
     ESP_REQUIRE(xh_numel >= n_shards * RG * 16 * K, "dense_prompt: xh needs n_shards * ceil(T / 16) * 16 * K halves");
     ESP_REQUIRE(wf_numel >= (int64_t)nbt * 128 * K, "dense_prompt: wf needs K * N halves");
-    const int64_t rot_units = n_shards * RG * (K / 128), dec_units = (int64_t)nbt * (K / 32) / PREP_WAVES;
+    const int64_t rot_units = n_shards * RG * (K / 128) * 16, rot_wgs = (rot_units + ROT_UNITS - 1) / ROT_UNITS, dec_units = (int64_t)nbt * (K / 32) / PREP_WAVES;
     ESP_REQUIRE(rot_units + dec_units < (int64_t(1) << 31) && (T + PG_ROWS) / PG_ROWS * nbt < (int64_t(1) << 28),
                 "dense_prompt: too many rows for one launch");
     p.n = a.n = (int)n_shards;
@@ -418,6 +398,8 @@ extern "C" int esp_dense_prompt(const void* x, int x_dtype, int64_t x_stride, in
     p.xh = static_cast<uint16_t*>(xh);
     p.wf = static_cast<uint16_t*>(wf);
     p.rot_units = (unsigned)rot_units;
+    p.rot_wgs = (unsigned)rot_wgs;
+    p.wide = rot_wide(x, x_stride, p.suh, (int)n_shards);
     a.scale = gemm_scale((int)cb);
     a.xh = static_cast<const uint16_t*>(xh);
     a.wf = static_cast<const uint16_t*>(wf);
@@ -433,7 +415,7 @@ extern "C" int esp_dense_prompt(const void* x, int x_dtype, int64_t x_stride, in
     switch (cb * 32 + k2) {
 #define ESP_PREP_CASE(CB_, K2_)                                                                              \
     case CB_ * 32 + K2_:                                                                                     \
-        prompt_prep_kernel<gemm_cb(CB_), K2_><<<(unsigned)(rot_units + dec_units), 256, 0, st>>>(p);         \
+        prompt_prep_kernel<gemm_cb(CB_), K2_><<<(unsigned)(rot_wgs + dec_units), 256, 0, st>>>(p);           \
         break;
         ESP_CASES(ESP_PREP_CASE)
 #undef ESP_PREP_CASE

@@ -230,25 +230,34 @@ class Dense:
             y[:, self.N:].zero_()                     # padding columns (the LM head's vocabulary padding)
         if x.stride(-1) != 1:
             x = x.contiguous()
+        for l in self.launches:
+            self._window(x, codes, pre, post, y, l)
+        return y
+
+    def _window(self, x, codes, pre, post, y, l) -> None:
+        """Launch l over the rows of x (at most MAX_ROWS) into its columns of y."""
         z, xh = scratch(x.device, 0, 0)
         e = ext()
         M = x.shape[0]
-        for l in self.launches:
-            pick = l.members
-            # a launch whose last split can poll the others' partials runs over the all-ones buffer (the same bits)
-            if OWN and polls(M, l.sk, l.w):
-                run, zl = e.dense_own, own_partials(x.device, l.sk * M * l.n)
-            else:
-                run, zl = e.dense, z
-            run(x, [codes[i] for i in pick], [pre[i] for i in pick], [post[i] for i in pick],
-                [self.col0[i] for i in pick], y, xh, zl, self.counters, l.k2, l.cb, l.sk, l.w, l.pf, ROT_SMEM)
-        return y
+        pick = l.members
+        # a launch whose last split can poll the others' partials runs over the all-ones buffer (the same bits)
+        if OWN and polls(M, l.sk, l.w):
+            run, zl = e.dense_own, own_partials(x.device, l.sk * M * l.n)
+        else:
+            run, zl = e.dense, z
+        run(x, [codes[i] for i in pick], [pre[i] for i in pick], [post[i] for i in pick], [self.col0[i] for i in pick],
+            y, xh, zl, self.counters, l.k2, l.cb, l.sk, l.w, l.pf, ROT_SMEM)
 
     def prompts(self) -> bool:
         """Whether forward_prompt takes this layer: 128-wide blocks, and no launch with too many weights to decode
         whole or with a K split shorter than its k slots."""
         return (self.K % 128 == 0 and all(m.out_features % 128 == 0 for m in self.mats) and
                 all(self.K * l.n <= PROMPT_WEIGHTS and l.sk * (l.w // 4) <= self.K // 32 for l in self.launches))
+
+    def _tile_is_window(self, T: int, launch) -> bool:
+        """Whether T rows of a launch in the tile mode run as one decode launch, whose sums are then esp_dense_tile's: no
+        K split and two k slots (the LM head, whose last row a prompt takes: 125 us as a 128-row tile, 72 as a window)."""
+        return T <= MAX_ROWS and launch.sk == 1 == tile_plan(self.K, launch.n) and launch.w == 4 * TILE_SLOTS
 
     def _tile_decodes_once(self, T: int, launch) -> bool:
         """Whether T rows of a launch in the tile mode run as esp_dense_prompt (the bits of esp_dense_tile, every weight
@@ -303,13 +312,16 @@ class Dense:
             y[:, self.N:].zero_()
         if x.stride(-1) != 1:
             x = x.contiguous()
-        if not all(self._tile_decodes_once(T, l) for l in self.launches):
+        if not all(self._tile_decodes_once(T, l) or self._tile_is_window(T, l) for l in self.launches):
             self.reserve_prompt(T)
         z, xh, cnt = prompt_scratch(x.device, 0, 0, 0)
         e = ext()
         for l in self.launches:
             pick = l.members
             sk = tile_plan(self.K, l.n)
+            if self._tile_is_window(T, l):
+                self._window(x, codes, pre, post, y, l)
+                continue
             if self._tile_decodes_once(T, l):
                 self._prompt(x, codes, pre, post, y, l, sk, TILE_SLOTS)
                 continue
