@@ -112,3 +112,33 @@ def test_grouped_prompt_refuses_bad_table_entries(dev, ext, table):
     assert bool(hit.any()) and not bool(hit.all())
     assert bool(torch.isnan(out[hit].float()).all()) and bool(torch.isfinite(out[~hit].float()).all())
     assert int(ext.status(True)) != 0
+
+
+@pytest.mark.parametrize("rows", [32, 64])
+@pytest.mark.parametrize("T,slots,E", [(1, 1, 3), (33, 9, 257), (517, 9, 257), (2048, 9, 257), (2100, 4, 17), (300, 8, 4096)])
+def test_group_tiles_equals_group_and_tile_list(dev, ext, T, slots, E, rows):
+    """One launch's tables against group's, and its list against the member counts: random picks, ids out of range among
+    them, an id twice a row, more picks than one batch of a workgroup (16384)."""
+    gen = torch.Generator().manual_seed(T + rows)
+    pick = torch.randint(-1, E + 1, (T, slots), generator=gen, dtype=torch.int32)
+    pick[::3, -1] = E - 1
+    pick = pick.reshape(-1).to(dev)
+    maxu, P = min(T * slots, E), T * slots
+    maxm = min(P, 2 * T)
+    cap = min(maxu * -(-maxm // rows), -(-P // rows) + maxu)
+
+    def tables():
+        return [torch.full(shape, -7, dtype=torch.int32, device=dev) for shape in ((maxu,), (1,), (maxu, maxm))]
+    (ids, count, members), (ids2, count2, members2) = tables(), tables()
+    tiles = torch.full((1 + cap,), -7, dtype=torch.int32, device=dev)
+    ext.group(pick, ids, count, members, T, slots, E)
+    ext.group_tiles(pick, ids2, count2, members2, T, slots, E, rows, tiles)
+    u = int(count.item())
+    assert int(count2.item()) == u and torch.equal(ids2[:u], ids[:u])
+    have = (members[:u] >= 0).sum(dim=1).tolist()
+    want = [i << 16 | t for i, h in enumerate(have) for t in range(-(-h // rows))]
+    assert tiles[:1 + len(want)].tolist() == [len(want)] + want
+    for i, h in enumerate(have):
+        full = min(-(-h // rows) * rows, maxm)
+        assert torch.equal(members2[i, :full], members[i, :full]), i
+    G.check_status()

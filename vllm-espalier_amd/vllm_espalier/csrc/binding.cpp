@@ -221,6 +221,43 @@ void down_combine(const at::Tensor& Z, const at::Tensor& pick, const at::Tensor&
                           mptr<float>(out), rows, P, D, SK, slots, E, cur_stream()));
 }
 
+// esp_group_tiles: group and tile_list of a whole prompt in one launch
+void group_tiles(const at::Tensor& pick, at::Tensor uids, at::Tensor ucount, at::Tensor members, int64_t R, int64_t slots,
+                 int64_t E, int64_t rows, at::Tensor tiles) {
+    for (const at::Tensor* t : std::initializer_list<const at::Tensor*>{&pick, &uids, &ucount, &members, &tiles})
+        check(*t, at::kInt, "int table");
+    TORCH_CHECK(pick.numel() >= R * slots, "pick too small");
+    TORCH_CHECK(members.dim() == 2 && members.size(0) >= uids.numel() && members.size(1) >= 1, "members too small");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(pick.device());
+    call(esp_group_tiles(cptr<int32_t>(pick), mptr<int32_t>(uids), uids.numel(), mptr<int32_t>(ucount),
+                         mptr<int32_t>(members), members.size(1), R, slots, E, rows, mptr<int32_t>(tiles), tiles.numel(),
+                         cur_stream()));
+}
+
+// esp_shared_slots: group_shared's pick / weight tables alone
+void shared_slots(const at::Tensor& pick_in, const at::Tensor& wts_in, const at::Tensor& x, int64_t x_stride,
+                  const c10::optional<at::Tensor>& gate_w, int64_t shared_id, at::Tensor pick_out, at::Tensor wts_out,
+                  int64_t R, int64_t slots_in) {
+    check(pick_in, at::kInt, "pick_in");
+    check(wts_in, at::kFloat, "wts_in");
+    check(pick_out, at::kInt, "pick_out");
+    check(wts_out, at::kFloat, "wts_out");
+    TORCH_CHECK(x.is_cuda() && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf),
+                "x: bf16/fp16 CUDA");
+    if (gate_w.has_value())
+        TORCH_CHECK(gate_w->scalar_type() == x.scalar_type() && gate_w->is_contiguous() && gate_w->numel() == x.size(1),
+                    "gate_w: x's dtype, [H]");
+    TORCH_CHECK(shared_id < 0 || gate_w.has_value(), "a shared slot needs its gate weight");
+    const int64_t slots = slots_in + (shared_id >= 0);
+    TORCH_CHECK(pick_in.numel() >= R * slots_in && wts_in.numel() >= R * slots_in && pick_out.numel() >= R * slots &&
+                    wts_out.numel() >= R * slots,
+                "pick / wts too small");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    call(esp_shared_slots(cptr<int32_t>(pick_in), cptr<float>(wts_in), x.data_ptr(), dtype_code(x), x_stride, x.size(1),
+                          gate_w.has_value() ? gate_w->data_ptr() : nullptr, shared_id, mptr<int32_t>(pick_out),
+                          mptr<float>(wts_out), R, slots_in, cur_stream()));
+}
+
 void group_shared(const at::Tensor& pick_in, const at::Tensor& wts_in, const at::Tensor& x, int64_t x_stride,
                   const c10::optional<at::Tensor>& gate_w, int64_t shared_id, at::Tensor pick_out, at::Tensor wts_out,
                   at::Tensor uids, at::Tensor ucount, at::Tensor members, int64_t R, int64_t slots_in, int64_t E) {
@@ -764,6 +801,8 @@ PYBIND11_MODULE(espalier_ext, m) {
     m.def("tile_list", &tile_list, py::arg("ucount"), py::arg("members"), py::arg("nexp_max"), py::arg("P"),
           py::arg("tiles"), py::arg("rows") = 32);
     m.def("grouped_prompt", &grouped_prompt);
+    m.def("group_tiles", &group_tiles);
+    m.def("shared_slots", &shared_slots);
     m.def("grouped_list", &grouped_list);
     m.def("dequant", &dequant);
     m.def("group", &group);

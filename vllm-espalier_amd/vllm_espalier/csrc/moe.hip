@@ -462,6 +462,95 @@ __global__ __launch_bounds__(GW) void group_wide_kernel(const int* __restrict__ 
     for (int m = tid; m < maxm; m += GW) members[at + m] = m < count ? mem_sh[m] : -1;
 }
 
+// ------------------------------------------------------------------------------------------------------------------
+// esp_group_tiles: the grouping of a whole prompt and its tile list in one launch, a workgroup an id. Every workgroup
+// counts all the picks by id in shared memory (so it knows its place, its first tile and the totals by itself) and ranks
+// its own id's picks in pick order: GL_PER consecutive picks a thread with their loads in flight, a scan over the threads
+// a batch. Tables as group_block's, but a member row is filled (-1 past its members) to a whole tile only. Latency-bound:
+// 13.8k picks of 257 ids, 26 us (a barrier every 256 picks) + 12 us for the list in a launch of one workgroup before.
+// ------------------------------------------------------------------------------------------------------------------
+constexpr int GL = 1024, GL_PER = 16;
+
+__global__ __launch_bounds__(GL) void group_tiles_kernel(const int* __restrict__ pick, int n, int slots, int nid, int maxm,
+                                                         int rows, int* __restrict__ uids, int* __restrict__ ucount,
+                                                         int* __restrict__ members, int* __restrict__ tiles, int cap) {
+    extern __shared__ int mem_sh[];                      // this id's member codes, in pick order
+    __shared__ int hist[MAX_GROUP_IDS];
+    __shared__ int wave_sum[GL / 64][4];
+    const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int i = tid; i < nid; i += GL) hist[i] = 0;
+    __syncthreads();
+    int count = 0;                                       // this id's picks so far (the same in every thread)
+    for (int base = 0; base < n; base += GL * GL_PER) {
+        const int i0 = base + tid * GL_PER;
+        int v[GL_PER];
+#pragma unroll
+        for (int j = 0; j < GL_PER; ++j) v[j] = i0 + j < n ? pick[i0 + j] : -1;
+        unsigned mine = 0u;
+#pragma unroll
+        for (int j = 0; j < GL_PER; ++j) {
+            if (v[j] >= 0 && v[j] < nid) atomicAdd(&hist[v[j]], 1);
+            mine |= (unsigned)(v[j] == e) << j;
+        }
+        const int c = __builtin_popcount(mine);
+        int incl = c;                                    // inclusive prefix over the wave
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += o;
+        }
+        if (lane == 63) wave_sum[wave][0] = incl;
+        __syncthreads();
+        int rank = count + incl - c, total = 0;
+#pragma unroll
+        for (int w = 0; w < GL / 64; ++w) {
+            const int t = wave_sum[w][0];
+            rank += w < wave ? t : 0;
+            total += t;
+        }
+        for (; mine != 0u; mine &= mine - 1, ++rank) {
+            const int i = i0 + __builtin_ctz(mine);
+            if (rank < maxm) mem_sh[rank] = (i / slots) * 32 + i % slots;
+        }
+        count += total;
+        __syncthreads();                                 // wave_sum is rewritten by the next batch
+    }
+    // over the ids: this one's place and first tile, the used ids and the tiles in all
+    int sums[4] = {0, 0, 0, 0};
+    for (int i = tid; i < nid; i += GL) {
+        const int h = hist[i] < maxm ? hist[i] : maxm, t = (h + rows - 1) / rows;
+        sums[0] += i < e && h > 0;
+        sums[1] += i < e ? t : 0;
+        sums[2] += h > 0;
+        sums[3] += t;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) sums[q] += __shfl_xor(sums[q], d, 64);
+        if (lane == 0) wave_sum[wave][q] = sums[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        sums[q] = 0;
+#pragma unroll
+        for (int w = 0; w < GL / 64; ++w) sums[q] += wave_sum[w][q];
+    }
+    if (e == 0 && tid == 0) {
+        *ucount = sums[2];
+        tiles[0] = sums[3] < cap ? sums[3] : cap;
+        if (sums[3] > cap) raise_status(ESP_STATUS_TILE_LIST);
+    }
+    if (count == 0) return;                              // the same in every thread
+    if (tid == 0) uids[sums[0]] = e;
+    const int have = count < maxm ? count : maxm, mt = (have + rows - 1) / rows;
+    const size_t at = (size_t)sums[0] * maxm;
+    for (int m = tid; m < mt * rows && m < maxm; m += GL) members[at + m] = m < have ? mem_sh[m] : -1;
+    for (int t = tid; t < mt; t += GL)
+        if (sums[1] + t < cap) tiles[1 + sums[1] + t] = (sums[0] << 16) | t;
+}
+
 // group_shared's pick / weight tables for any number of rows, a wave a row: the routed slots copied, the shared slot
 // added with weight sigmoid(x . gate_w) computed exactly as group_shared_kernel does (the same bits)
 __global__ __launch_bounds__(256) void shared_slots_kernel(const int* __restrict__ pick_in, const float* __restrict__ wts_in,
@@ -1998,6 +2087,40 @@ extern "C" int esp_grouped(const void* X0, const void* X1, const int64_t* TP0, c
     (void)pf;
     return grouped_impl(X0, X1, TP0, TP1, B0, B1, C0, C1, uids, nexp_max, ucount, members, maxm, Z, z_numel, mats, K,
                         N, P, SK, slots, warps, lo, hi, nullptr, stream);
+}
+
+extern "C" int esp_group_tiles(const int32_t* pick, int32_t* uids, int64_t maxu, int32_t* ucount, int32_t* members,
+                               int64_t maxm, int64_t R, int64_t slots, int64_t E, int64_t rows, int32_t* tiles,
+                               int64_t tiles_numel, void* stream) {
+    ESP_REQUIRE(pick && uids && ucount && members && tiles, "group_tiles: null pointer");
+    ESP_REQUIRE(E >= 1 && E <= MAX_GROUP_IDS, "too many experts for the grouping kernel");
+    ESP_REQUIRE(slots >= 1 && slots <= 32, "at most 32 slots a row");
+    ESP_REQUIRE(R >= 1 && R * slots <= (int64_t(1) << 24), "grouping window too large");
+    ESP_REQUIRE(maxu >= (R * slots < E ? R * slots : E), "uids too small");
+    ESP_REQUIRE(maxm >= 1 && maxm <= 11264, "group_tiles: at most 11264 members an expert");      // 44 KiB beside the counts
+    ESP_REQUIRE(rows == 32 || rows == 64, "tile_list: tiles of 32 or 64 members");
+    const int64_t cap = tile_list_cap(R * slots < E ? R * slots : E, maxm, R * slots, rows);
+    ESP_REQUIRE(tiles_numel >= 1 + cap, "group_tiles: tiles needs 1 + min(U * ceil(maxm / rows), ceil(P / rows) + U) ints "
+                                        "(P = R * slots picks, U = min(P, E) expert slots)");
+    group_tiles_kernel<<<(unsigned)E, GL, (size_t)maxm * 4, (hipStream_t)stream>>>(
+        pick, (int)(R * slots), (int)slots, (int)E, (int)maxm, (int)rows, uids, ucount, members, tiles, (int)cap);
+    return esp_host::launch_check("group_tiles");
+}
+
+extern "C" int esp_shared_slots(const int32_t* pick_in, const float* wts_in, const void* x, int x_dtype, int64_t x_stride,
+                                int64_t H, const void* gate_w, int64_t shared_id, int32_t* pick_out, float* wts_out,
+                                int64_t R, int64_t slots_in, void* stream) {
+    const int64_t has = shared_id >= 0 ? 1 : 0;
+    ESP_REQUIRE(pick_in && wts_in && pick_out && wts_out, "shared_slots: null pointer");
+    ESP_REQUIRE(slots_in >= 1 && slots_in + has <= 32 && R >= 1 && R * (slots_in + has) <= (int64_t(1) << 24),
+                "shared_slots: at most 32 slots a row");
+    ESP_REQUIRE(!has || (gate_w && x), "a shared slot needs its gate weight");
+    ESP_REQUIRE(!has || (x_dtype == ESP_BF16 || x_dtype == ESP_F16), "x: bf16/fp16");
+    ESP_REQUIRE(!has || (H % 256 == 0 && x_stride % 4 == 0), "shared_slots: H must be a multiple of 256");
+    shared_slots_kernel<<<(unsigned)((R + 3) / 4), 256, 0, (hipStream_t)stream>>>(
+        pick_in, wts_in, static_cast<const uint16_t*>(x), (int)x_stride, x_dtype == ESP_BF16,
+        static_cast<const uint16_t*>(gate_w), (int)H, (int)shared_id, pick_out, wts_out, (int)R, (int)slots_in);
+    return esp_host::launch_check("shared_slots");
 }
 
 extern "C" int esp_tile_list_rows(const int32_t* ucount, const int32_t* members, int64_t nexp_max, int64_t maxm,

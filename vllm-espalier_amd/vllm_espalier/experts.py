@@ -501,7 +501,7 @@ def prefill_scratch(layer: Layer, rows: int, slots: int, device) -> PrefillScrat
     return found.handed_out()
 
 
-PREFILL_MAX_ROWS = 16384    # tokens one whole-prompt grouping takes (the wide grouping's members an expert)
+PREFILL_MAX_ROWS = 8192     # tokens one whole-prompt pass takes (esp_group_tiles keeps an expert's members in shared memory)
 
 
 def prefill(x: torch.Tensor, pick: torch.Tensor | None, wts: torch.Tensor | None, L: Layer, s: PrefillScratch,
@@ -542,16 +542,14 @@ def _prefill(x, pick, wts, L: Layer, s: PrefillScratch, k: int, gate, out, out_s
         if gate is None:
             raise ValueError("prefill needs the picks or the router weight")
         e.route_rows(x, gate, L.gate_w, k, L.shared_id, s.logits, pick_p, wts_p)
-        e.group(pick_p, ids, s.count, members, T, slots, L.E)
     else:
-        e.group_shared(pick, wts, x, x.stride(0), L.gate_w, L.shared_id, pick_p, wts_p, ids, s.count, members, T, k,
-                       L.E)
+        e.shared_slots(pick, wts, x, x.stride(0), L.gate_w, L.shared_id, pick_p, wts_p, T, k)
+    # the expert launches run over the grouping's non-empty (expert, member tile) pairs only: a grid of every expert slot
+    # times every member tile is mostly empty workgroups
+    tr = tile_rows(T, k, L.E - has_shared)
+    e.group_tiles(pick_p, ids, s.count, members, T, slots, L.E, tr, s.tiles)
     e.rot_in(x, x.stride(0), pick_p, L.suh_g, L.suh_u, s.xg, s.xu, T, L.D, slots, L.E)
     t, b, c = L.ptr[2], L.k2[2], L.cb[2]
-    # over the grouping's non-empty (expert, member tile) pairs only: a grid of every expert slot times every member tile
-    # is mostly empty workgroups
-    tr = tile_rows(T, k, L.E - has_shared)
-    e.tile_list(s.count, members, ids.numel(), P, s.tiles, tr)
     e.grouped_prompt(s.xg, s.xu, L.ptr[0], L.ptr[1], L.k2[0], L.k2[1], L.cb[0], L.cb[1], ids, s.count, members, s.tiles,
                      tr, s.z, 2, L.D, L.I, P, sk_gu, slots, *L.k2_gu)
     e.gateup_epilogue(s.z, pick_p, L.svh_g, L.svh_u, L.suh_d, s.xd, T, P, L.I, 1, slots, L.E, math.inf, ACT_F32)
