@@ -164,7 +164,7 @@ __device__ __forceinline__ void block_gemm(const uint32_t* __restrict__ T, int N
             for (int g = 0; g < MG; ++g) aload(g, k0 + 32 * (first + st), av[g]);
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                const f16x8 b = __builtin_bit_cast(f16x8, decode_words<CB, K2>(w[j], lp));
+                const f16x8 b = decode_b<CB, K2>(w[j], lp);
 #pragma unroll
                 for (int g = 0; g < MG; ++g)
                     acc[j][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[g], b, acc[j][g], 0, 0, 0);
@@ -204,7 +204,7 @@ __device__ __forceinline__ void decode_ahead(const uint32_t* stage_lds, int kr, 
 #pragma unroll
                 for (int q = 0; q < 6; ++q) w[j][q] = tl[j * TW + lw.off[q]];
 #pragma unroll
-            for (int j = 0; j < 2; ++j) pb.b[i][j] = decode_words<CB, K2>(w[j], lp);
+            for (int j = 0; j < 2; ++j) pb.b[i][j] = __builtin_bit_cast(u32x4, decode_b<CB, K2>(w[j], lp));
         }
     }
 }

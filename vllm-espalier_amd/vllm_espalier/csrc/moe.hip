@@ -814,7 +814,7 @@ __device__ __forceinline__ void grouped_body_staged(const GroupedArgs& a, const 
             for (int g = 0; g < MG; ++g) al(g, 32 * ls, av[g]);
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                const f16x8 b = __builtin_bit_cast(f16x8, decode_words<CB, K2>(w[j], lp));
+                const f16x8 b = decode_b<CB, K2>(w[j], lp);
 #pragma unroll
                 for (int g = 0; g < MG; ++g)
                     acc[j][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[g], b, acc[j][g], 0, 0, 0);

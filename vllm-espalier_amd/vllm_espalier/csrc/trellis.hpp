@@ -103,11 +103,13 @@ __device__ __forceinline__ uint32_t mcg_hash(uint32_t s) { return (s * MCG_MUL &
 // mcg values of two states as packed fp16 (lo = s0): the two halves of each hash added in one RNE fp16 add
 // (experts_grouped.cuh:64-79). Two v_add_f16 reading the halves through SDWA, the second writing the high half of the
 // result and keeping its low half: two instructions a pair, where gathering the halves for one packed add takes three.
+// Inline asm here and below works in place, in a register that the compiler's own instruction has just written: it may be
+// one whose old value an MFMA in flight still reads (its C operand, read last), and the compiler sets the wait that this
+// needs before its own writes only.
 __device__ __forceinline__ uint32_t mcg_pair(uint32_t s0, uint32_t s1) {
-    const uint32_t x0 = mcg_hash(s0), x1 = mcg_hash(s1);
-    uint32_t d;
-    asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1"
-        : "=v"(d) : "v"(x0));
+    uint32_t d = mcg_hash(s0);
+    const uint32_t x1 = mcg_hash(s1);
+    asm("v_add_f16_sdwa %0, %0, %0 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1" : "+v"(d));
     asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1"
         : "+v"(d) : "v"(x1));
     return d;
@@ -123,9 +125,7 @@ __device__ __forceinline__ _Float16 mcg_one(uint32_t s) {
 // f32(v) * k with one rounding, v read as fp16 by v_fma_mix_f32 (no separate conversion); the +0 addend leaves every
 // product unchanged (v is never -0: the sum of two opposite halves is +0)
 __device__ __forceinline__ float mul_mix(_Float16 v, float k) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(v), "v"(k));
-    return r;
+    return __builtin_fmaf((float)v, k, 0.f);
 }
 
 // Codebook value pair. CB: 1 mcg; 3 E2M1 snap; 6 / 7 fp16(q * c) on the int5 / int6 grid; the GEMM forms (gemm_cb):
@@ -142,19 +142,17 @@ __device__ __forceinline__ uint32_t decode_pair(uint32_t s0, uint32_t s1) {
         // more apart, relative). Back to fp16 through the same instruction pair, then * 0.75 (exact).
         const float k = E2M1_K;
         const float y0 = mul_mix(mcg_one(s0), k), y1 = mul_mix(mcg_one(s1), k);   // no packing of the two values
-        // the conversion writes byte 0 of code and keeps the other three, which nothing reads: an output operand
-        uint32_t code, h;
-        asm("v_cvt_scalef32_pk_fp4_f32 %0, %1, %2, %3" : "=v"(code) : "v"(y0), "v"(y1), "v"(1.0f));
-        asm("v_cvt_scalef32_pk_f16_fp4 %0, %1, %2" : "=v"(h) : "v"(code), "v"(1.0f));
+        // the conversion writes byte 0 of its first operand and keeps the other three, which nothing reads
+        const uint32_t code = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(__builtin_bit_cast(uint32_t, y0), y0, y1, 1.0f, 0);
+        const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(code, 1.0f, 0));
         if constexpr (CB == 19) return h;                  // the unscaled grid: the GEMM scales its sums by 0.75
         const f16x2 q = __builtin_bit_cast(f16x2, h) * f16x2{(_Float16)0.75f, (_Float16)0.75f};
         return __builtin_bit_cast(uint32_t, q);
     } else if constexpr (CB == 23) {
-        uint32_t d;                                      // the high half is written next, by v_fma_mixhi_f16
-        const float k = GRID_K6M, m = GRID_MAGIC;
-        asm("v_fma_mixlo_f16 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(d) : "v"(mcg_one(s0)), "v"(k), "v"(m));
-        asm("v_fma_mixhi_f16 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "+v"(d) : "v"(mcg_one(s1)), "v"(k), "v"(m));
-        const f16x2 q = __builtin_bit_cast(f16x2, d) - f16x2{(_Float16)GRID_MAGIC, (_Float16)GRID_MAGIC};   // exact
+        const float k = GRID_K6M, m = GRID_MAGIC;         // v_fma_mixlo_f16 and v_fma_mixhi_f16
+        const f16x2 d = {(_Float16)__builtin_fmaf((float)mcg_one(s0), k, m),
+                         (_Float16)__builtin_fmaf((float)mcg_one(s1), k, m)};
+        const f16x2 q = d - f16x2{(_Float16)GRID_MAGIC, (_Float16)GRID_MAGIC};   // exact
         return __builtin_bit_cast(uint32_t, q);
     } else {
         static_assert(CB == 6 || CB == 7 || CB == 22, "codebook");
@@ -190,9 +188,14 @@ __device__ __forceinline__ u32x4 decode_words(const uint32_t (&w)[6], const Lane
     return v;
 }
 
+// The same as an MFMA's B operand. An MFMA may read a register only two wait states after a vector instruction wrote it;
+// the compiler keeps that for its own instructions, but the mcg values' last writes are inline asm (with one state between,
+// 8-bit tiles of a kernel that read its words ahead came out wrong).
 template <int CB, int K2>
 __device__ __forceinline__ f16x8 decode_b(const uint32_t (&w)[6], const LanePlan<K2>& lp) {
-    return __builtin_bit_cast(f16x8, decode_words<CB, K2>(w, lp));
+    u32x4 v = decode_words<CB, K2>(w, lp);
+    if constexpr (CB == 1) asm("s_nop 1" : "+v"(v));
+    return __builtin_bit_cast(f16x8, v);
 }
 
 // fp16 bits of B slot i (0..7) of a decoded operand
