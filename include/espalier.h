@@ -108,6 +108,17 @@ int esp_dense_tile(const void* x, int x_dtype, int64_t x_stride, int64_t T, int6
                    int64_t xh_numel, float* Z, int64_t z_numel, int32_t* counters, int64_t counters_numel, int64_t k2,
                    int64_t cb, int64_t SK, void* stream);
 
+/* dense of one matrix over a few rows (M at most 6) with its column blocks cut into equal shares for the workgroups the
+ * device holds (no reference counterpart): the bits of esp_dense at SK = 1, W = 8, for layers of more blocks than that. x,
+ * y (at the matrix's first column) as esp_dense; K a multiple of 256. With norm_w the rows are RMSNorm(x + d1 + d2) *
+ * norm_w and the residual goes to h_out, as esp_dense_rmsnorm (M at most 2; d1 / d2 may be null). part fp32 scratch: 256
+ * floats a row and workgroup (two a compute unit, at most one a 128-column block), all-ones on entry and left so, as
+ * esp_dense_own's partials. A wait past ~20 ms sets ESP_STATUS_WAIT_TIMEOUT. */
+int esp_dense_stream(const void* x, int x_dtype, int64_t x_stride, int64_t M, int64_t K, const void* trellis,
+                     const void* suh, const void* svh, int64_t N, void* y, int y_dtype, int64_t y_stride, const void* d1,
+                     const void* d2, const void* norm_w, double eps, void* h_out, float* part, int64_t part_numel,
+                     int64_t k2, int64_t cb, void* stream);
+
 /* dense over a prompt of any number of rows with every weight decoded once (no reference counterpart): the rows rotated
  * into xh and the weights decoded to fp16 into wf, then a GEMM on those fragments whose sums keep the order of a launch
  * with K splits SK and KW k slots: the bits of esp_dense at that SK and W = 4 * KW, or of esp_dense_tile at that SK

@@ -113,3 +113,70 @@ def test_tile_mode_few_rows_of_a_wide_layer(dev):
     y = d.forward_tile(x)
     for T in (1, 7, 32):
         assert torch.equal(d.forward_tile(x[:T]), y[:T]), T
+
+
+@pytest.mark.parametrize("M", [1, 2, 5, 6])
+@pytest.mark.parametrize("K,blocks,bits,grid", [(256, 600, 2, "mcg"), (1024, 260, 4, "int6"), (2048, 517, 6, "mcg"),
+                                                (768, 1187, 3, "int5"), (512, 513, 5, "mcg"), (1280, 700, 8, "mcg")])
+def test_stream_equals_one_workgroup_a_block(dev, ext, monkeypatch, K, blocks, bits, grid, M):
+    """esp_dense_stream against esp_dense: shares that end inside blocks, blocks of one stage, as many blocks as workgroups;
+    launches in a row, the hand-off buffer left all-ones and no wait timed out."""
+    gen = torch.Generator(device=dev).manual_seed(K + blocks)
+    d = D.Dense([WL.matrix(K, 128 * blocks, bits, grid, gen, dev)])
+    l = d.launches[0]
+    if not d._streams(M, l):
+        pytest.skip("the rows do not leave two workgroups a CU")
+    for dtype in (torch.bfloat16, torch.float16):
+        x = _rows(M, K, dtype, dev, M)
+        monkeypatch.setattr(D, "STREAM", False)
+        want = d.forward(x)
+        monkeypatch.setattr(D, "STREAM", True)
+        for _ in range(3):
+            assert torch.equal(d.forward(x), want)
+    assert bool((d._stream_part(dev).view(torch.int32) == -1).all())
+    assert int(ext.status(True)) == 0
+
+
+@pytest.mark.parametrize("M", [1, 2])
+def test_stream_rmsnorm_equals_dense_rmsnorm(dev, monkeypatch, M):
+    gen = torch.Generator(device=dev).manual_seed(9)
+    d = D.Dense([WL.matrix(2048, 128 * 530, 4, "mcg", gen, dev)])
+    assert d.norm_fusable(M) and d._streams(M, d.launches[0])
+    h, d1, d2 = (_rows(M, d.K, torch.bfloat16, dev, s) for s in (1, 2, 3))
+    w = (1 + 0.1 * torch.randn((d.K,), generator=torch.Generator().manual_seed(4))).to(torch.bfloat16).to(dev)
+    outs = []
+    for stream in (False, True):
+        monkeypatch.setattr(D, "STREAM", stream)
+        h_out, y = torch.zeros_like(h), torch.empty((M, d.n_out), dtype=h.dtype, device=dev)
+        d.forward_rmsnorm(h, d1, d2, w, 1e-6, h_out, y)
+        d.forward_rmsnorm(h, None, None, w, 1e-6, torch.zeros_like(h), y.clone())
+        outs.append((h_out, y))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+def test_stream_graph_replay(dev):
+    gen = torch.Generator(device=dev).manual_seed(10)
+    d = D.Dense([WL.matrix(1024, 128 * 700, 4, "mcg", gen, dev)])
+    x = _rows(1, d.K, torch.bfloat16, dev, 1)
+    want = d.forward(x)
+    calls = D.STREAM_SPARES + 2                                # the last ones fill their buffer in the graph
+    y = torch.empty((calls, *want.shape), dtype=want.dtype, device=dev)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        for i in range(calls):
+            d.forward(x, out=y[i])
+    for i in range(4):
+        y.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(v, want) for v in y), i
+        assert torch.equal(d.forward(x), want)                 # eager work between replays
+    side = torch.cuda.Stream()                                 # another stream, another hand-off buffer
+    own = d._stream_part(dev)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        assert d._stream_part(dev).data_ptr() != own.data_ptr()
+        ys = [d.forward(x) for _ in range(3)]
+    ym = [d.forward(x) for _ in range(3)]
+    torch.cuda.synchronize()
+    assert all(torch.equal(v, want) for v in ys + ym)

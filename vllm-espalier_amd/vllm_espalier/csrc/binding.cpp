@@ -360,6 +360,39 @@ void dense_own(const at::Tensor& x, const std::vector<at::Tensor>& T, const std:
     dense_call(x, T, suh, svh, col0, y, xh, Z, counters, k2, cb, SK, W, PF, rot_smem, true);
 }
 
+// dense of one wide matrix over a few rows (esp_dense_stream; no reference counterpart)
+void dense_stream(const at::Tensor& x, const c10::optional<at::Tensor>& d1, const c10::optional<at::Tensor>& d2,
+                  const c10::optional<at::Tensor>& norm_w, double eps, const c10::optional<at::Tensor>& h_out,
+                  const at::Tensor& T, const at::Tensor& suh, const at::Tensor& svh, int64_t col0, at::Tensor y,
+                  at::Tensor part, int64_t k2, int64_t cb) {
+    TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1, "x: CUDA [M, K], unit column stride");
+    TORCH_CHECK(y.is_cuda() && y.dim() == 2 && y.stride(1) == 1 && y.size(0) >= x.size(0),
+                "y: CUDA [M, N], unit column stride");
+    TORCH_CHECK(T.is_cuda() && T.scalar_type() == at::kShort && T.is_contiguous() && T.dim() == 3,
+                "trellis: contiguous int16 [K/16, N/16, 16K]");
+    check(suh, at::kHalf, "suh");
+    check(svh, at::kHalf, "svh");
+    check(part, at::kFloat, "part");
+    const int64_t K = x.size(1), N = svh.numel();
+    TORCH_CHECK(T.size(0) * 16 == K && T.size(1) * 16 == N && T.size(2) == 8 * k2 && suh.numel() == K, "matrix shape");
+    TORCH_CHECK(col0 >= 0 && col0 % 4 == 0 && col0 + N <= y.size(1), "matrix columns past y");
+    if (norm_w.has_value()) {
+        TORCH_CHECK(x.is_contiguous() && h_out.has_value(), "a norm takes contiguous rows and h_out");
+        for (const c10::optional<at::Tensor>* t : {&d1, &d2, &h_out})
+            TORCH_CHECK(!t->has_value() || ((*t)->is_contiguous() && (*t)->scalar_type() == x.scalar_type() &&
+                                            (*t)->sizes() == x.sizes()),
+                        "d1 / d2 / h_out: x's dtype and shape");
+        check(*norm_w, x.scalar_type(), "norm_w");
+        TORCH_CHECK(norm_w->numel() == K, "norm_w: [K]");
+    }
+    auto ptr = [](const c10::optional<at::Tensor>& t) { return t.has_value() ? t->data_ptr() : nullptr; };
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    call(esp_dense_stream(x.data_ptr(), dtype_code(x), x.stride(0), x.size(0), K, T.data_ptr(), suh.data_ptr(),
+                          svh.data_ptr(), N, static_cast<char*>(y.data_ptr()) + col0 * y.element_size(), dtype_code(y),
+                          y.stride(0), ptr(d1), ptr(d2), ptr(norm_w), eps, ptr(h_out), mptr<float>(part), part.numel(), k2,
+                          cb, cur_stream()));
+}
+
 // The matrices of a prompt launch, checked, as the C entry points take them
 struct PromptMats {
     std::vector<const void*> tp, sp, vp;
@@ -794,6 +827,7 @@ PYBIND11_MODULE(espalier_ext, m) {
     m.def("route_rows", &route_rows);
     m.def("dense_tile", &dense_tile);
     m.def("dense_prompt", &dense_prompt);
+    m.def("dense_stream", &dense_stream);
     m.def("dense", &dense);
     m.def("group_shared", &group_shared);
     m.def("down_combine2", &down_combine2);

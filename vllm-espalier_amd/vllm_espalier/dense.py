@@ -81,6 +81,13 @@ PROMPT_WEIGHTS = 1 << 27     # weights a launch decodes whole (2 bytes each)
 OWN = env("ESPALIER_DENSE_OWN", "1") != "0"
 
 
+STREAM_MAX_ROWS = 6          # rows of esp_dense_stream (2 with the norm inside)
+STREAM_PARTS = 16            # HIP streams of which a layer keeps a hand-off buffer (3 MiB)
+STREAM_SPARES = 4            # captured launches that get one filled beforehand (a fill in the graph: 6 us a replay)
+# wide launches over a few rows run as esp_dense_stream (the same bits); ESPALIER_DENSE_STREAM=0 runs them as esp_dense
+STREAM = env("ESPALIER_DENSE_STREAM", "1") != "0"
+
+
 class _SharedScratch:
     """The split-K partials Z (fp32) and the unfused rotation's rows xh (fp16), one pair a device, shared by every
     layer (layers run one after another). Sizes only grow. A pair that a growth replaces is kept for good only when a
@@ -197,6 +204,10 @@ class Dense:
         self.counters = torch.zeros(COUNTER_STRIDE * blocks, dtype=torch.int32, device=device)
         scratch(device, max(l.sk * MAX_ROWS * l.n for l in self.launches), 4 * MAX_ROWS * self.K)
         own_partials(device, max(l.sk * 2 * l.w // max(l.sk - 1, 1) * l.n for l in self.launches))
+        # esp_dense_stream's hand-off buffers: a HIP stream's own, spare ones for captured launches, and those in graphs
+        self._stream_parts, self._stream_graphs = {}, []
+        streams = any(self._streams(1, l) for l in self.launches)
+        self._stream_spare = list(self._new_parts(device, STREAM_SPARES)) if streams else []
 
     def _code(self, i: int) -> tuple[int, int]:
         m = self.mats[i]
@@ -234,8 +245,46 @@ class Dense:
             self._window(x, codes, pre, post, y, l)
         return y
 
+    def _streams(self, M: int, l) -> bool:
+        """Whether launch l over M rows runs as esp_dense_stream (its plan's bits): one matrix of more column blocks than
+        CUs in one K split (an LM head), and rows that leave two workgroups a CU. 2048 -> 151936, graph replays: 6 bits
+        (mcg) 73.1 us as a workgroup a block and 66.1 streamed at one row, 76.8 and 67.9 at four; 4 bits (int6) 77.7 and
+        73.2, 106.9 and 76.4."""
+        blocks = l.n // 128
+        smem = 4096 * l.k2 + M * (2 * self.K + 16 + 1024)
+        return (STREAM and 1 <= M <= STREAM_MAX_ROWS and len(l.members) == 1 and l.sk == 1 and l.w == 4 * TILE_SLOTS and
+                self.K % 256 == 0 and self.K * l.n <= 1 << 33 and l.n < 1 << 24 and blocks > 256 and
+                smem <= 80 * 1024 - 512)
+
+    def _new_parts(self, device, n: int):
+        floats = 2 * _cu_count(device) * 256 * STREAM_MAX_ROWS
+        return torch.full((n, floats), -1, dtype=torch.int32, device=device).view(torch.float32).unbind()
+
+    def _stream_part(self, device):
+        """The all-ones hand-off buffer for an esp_dense_stream launch on the current HIP stream, left all-ones by every
+        launch: launches on one stream run one after another, and no two streams share one. A captured launch has one of
+        its own, since a graph replays on any stream: a spare one, kept with the layer, or one filled in the graph. None
+        past STREAM_PARTS streams."""
+        if torch.cuda.is_current_stream_capturing():
+            try:
+                part = self._stream_spare.pop()
+            except IndexError:
+                return self._new_parts(device, 1)[0]
+            self._stream_graphs.append(part)
+            return part
+        key = torch.cuda.current_stream(device).cuda_stream
+        part = self._stream_parts.get(key)
+        if part is None and len(self._stream_parts) < STREAM_PARTS:
+            part = self._stream_parts.setdefault(key, self._new_parts(device, 1)[0])
+        return part
+
     def _window(self, x, codes, pre, post, y, l) -> None:
         """Launch l over the rows of x (at most MAX_ROWS) into its columns of y."""
+        if self._streams(x.shape[0], l) and (part := self._stream_part(x.device)) is not None:
+            i = l.members[0]
+            ext().dense_stream(x, None, None, None, 0.0, None, codes[i], pre[i], post[i], self.col0[i], y, part, l.k2,
+                               l.cb)
+            return
         z, xh = scratch(x.device, 0, 0)
         e = ext()
         M = x.shape[0]
@@ -342,9 +391,14 @@ class Dense:
     def forward_rmsnorm(self, h, d1, d2, norm_w, eps: float, h_out, out):
         """forward(RMSNorm(h + d1 + d2) * norm_w) with the residual h + d1 + d2 stored to h_out, the norm made inside
         the launch (bit-identical to add_rmsnorm then forward). h, d1, d2: [M, K] contiguous, the model's dtype."""
-        z, _ = scratch(h.device, 0, 0)
         l = self.launches[0]
         ms = [self.mats[i] for i in l.members]
+        if self._streams(h.shape[0], l) and (part := self._stream_part(h.device)) is not None:
+            m = ms[0]
+            ext().dense_stream(h, d1, d2, norm_w, eps, h_out, m.trellis, m.suh, m.svh, self.col0[l.members[0]], out,
+                               part, l.k2, l.cb)
+            return out
+        z, _ = scratch(h.device, 0, 0)
         ext().dense_rmsnorm(h, d1, d2, norm_w, eps, h_out, [m.trellis for m in ms], [m.suh for m in ms],
                             [m.svh for m in ms], [self.col0[i] for i in l.members], out, z, self.counters, l.k2, l.cb,
                             l.sk, l.w, ROT_SMEM)
