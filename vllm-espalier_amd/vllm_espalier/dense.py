@@ -350,8 +350,8 @@ class Dense:
 
     def forward_tile(self, x, trellis=None, suh=None, svh=None, out=None):
         """x [T, K], any T (a prompt) -> [T, n_out] in x's dtype, each weight decoded once for every 128 rows
-        (esp_dense_tile) or once (esp_dense_prompt, the same bits). A row's bits are its own (the same at any T), not those of forward. trellis / suh / svh:
-        lists that replace the matrices' own tensors, as in forward."""
+        (esp_dense_tile) or once (esp_dense_prompt, the same bits). A row's bits are its own (the same at any T), not
+        those of forward. trellis / suh / svh: lists that replace the matrices' own tensors, as in forward."""
         codes = trellis or [m.trellis for m in self.mats]
         pre = suh or [m.suh for m in self.mats]
         post = svh or [m.svh for m in self.mats]
