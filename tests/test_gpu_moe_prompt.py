@@ -60,6 +60,19 @@ def test_windows_whole_prompt_equals_windows(dev, monkeypatch, shape, T, rows):
     G.check_status()
 
 
+@pytest.mark.parametrize("plan", ["8,4", "16,4", "4,4;8,4", "8,4;4,4"])
+def test_windows_keep_decode_bits_under_a_forced_plan(dev, monkeypatch, plan):
+    """A forced plan of 8 or 16 waves sums several k slots a split: a prompt's tokens, a window's and those of one to four
+    rows still have the same bits."""
+    monkeypatch.setenv("ESPALIER_GROUPED_TILE_PLAN", plan)
+    L, router, k, s = _layer("wide", dev)
+    x = _x(70, L.D, dev, 11)
+    want = _by_window(x, None, None, L, s, k, router)
+    _same(G.windows(x, None, None, L, s, k=k, gate=router), want)
+    for n in (1, 3, 4, 5):
+        _same(G.windows(x[:n], None, None, L, s, k=k, gate=router), [t[:n] for t in want])
+
+
 def test_windows_given_picks_and_chunks(dev, monkeypatch):
     """vLLM's picks handed in, and a prompt of several passes."""
     monkeypatch.setattr(G, "WINDOWS_PROMPT_ROWS", 64)

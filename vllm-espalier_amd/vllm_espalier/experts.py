@@ -234,6 +234,8 @@ class Scratch:
         self.rows, self.slots, self.E = rows, slots, E
         self.cfg_gu = tile_config(D, I, True)
         self.cfg_d = tile_config(I, D, False)
+        # 4 waves a workgroup: one k slot a split, the only order of sums of the chained and the whole-prompt launches
+        self.one_slot = self.cfg_gu[1] == 4 and self.cfg_d[1] == 4
         P = rows * slots
         maxu = min(P, E)
         partials = P * max(2 * self.cfg_gu[2] * I, self.cfg_d[2] * D)
@@ -387,7 +389,8 @@ def routed2(x: torch.Tensor, pick: torch.Tensor | None, wts: torch.Tensor | None
         out_shared = torch.empty((R, L.D), dtype=x.dtype, device=x.device)
     shared_out = out_shared if has_shared else None
     sk_gu, sk_d = s.cfg_gu[2], s.cfg_d[2]
-    if CHAIN and FUSED and R <= CHAIN_ROWS and (L.D // sk_gu) % 128 == 0 and sk_d * 128 == L.I and L.I <= 1024:
+    if (CHAIN and FUSED and R <= CHAIN_ROWS and s.one_slot and (L.D // sk_gu) % 128 == 0 and sk_d * 128 == L.I and
+            L.I <= 1024):
         (tg, tu, td), (bg, bu, bd), (cg, cu, cd) = L.ptr, L.k2, L.cb
         e.moe_chain(x, x.stride(0), L.suh_g, L.suh_u, tg, tu, td, bg, bu, bd, cg, cu, cd, ids, s.count, members,
                     pick_p, wts_p, L.svh_g, L.svh_u, L.suh_d, L.svh_d, s.xdc, s.z, s.zd, s.y, out, shared_out,
@@ -419,11 +422,11 @@ def windows(x: torch.Tensor, pick: torch.Tensor | None, wts: torch.Tensor | None
             k: int | None = None, gate: torch.Tensor | None = None):
     """routed2 over any number of tokens (prefill), each exactly as in decode; with gate (and pick=None), route() first.
     More than s.rows tokens run as whole-prompt passes (experts.prefill's launches with the window launches' K splits, so
-    their bits: each picked expert decoded once for up to 64 of its tokens instead of once a window), or as consecutive
-    windows of s.rows tokens. Returns (routed sum, shared output or None)."""
+    their bits: each picked expert decoded once for up to 64 of its tokens instead of once a window), or, under a forced plan
+    of more waves (several k slots a split, which those launches do not sum), as consecutive windows of s.rows tokens. Returns (routed sum, shared output or None)."""
     out = torch.empty_like(x)
     shared_out = torch.empty_like(x) if L.shared_id >= 0 else None
-    whole = x.shape[0] > s.rows and (pick is not None or gate is not None) and _whole_prompt(x, L, gate)
+    whole = x.shape[0] > s.rows and (pick is not None or gate is not None) and s.one_slot and _whole_prompt(x, L, gate)
     step = min(WINDOWS_PROMPT_ROWS, _listed_rows(L)) if whole else s.rows
     for r0 in range(0, x.shape[0], step):
         rows = slice(r0, r0 + step)
