@@ -112,6 +112,46 @@ def test_windows_graph_outlives_a_longer_prompt(dev):
         torch.randn((256, 256), device=dev).sum()             # eager work between replays
 
 
+@pytest.mark.parametrize("mode", ["windows", "prefill"])
+def test_outgrown_prompt_scratch_outlives_its_streams(dev, mode):
+    """A prompt scratch allocated on stream a, used on b and outgrown there while b still has that prompt to run: a's next
+    allocations of the same sizes get other memory, and b's results are right."""
+    L, router, k, s = _layer("wide", dev)
+    slots = k + 1
+
+    def run(x):
+        if mode == "windows":
+            return G.windows(x, None, None, L, s, k=k, gate=router)
+        return G.prefill(x, None, None, L, G.prefill_scratch(L, x.shape[0], slots, dev), k, gate=router)
+
+    def held():
+        return s.prompt if mode == "windows" else G._PREFILL[(L.E, L.D, L.I, slots, str(dev))]
+    if mode == "prefill":
+        G._PREFILL.pop((L.E, L.D, L.I, slots, str(dev)), None)
+    x, longer = _x(50, L.D, dev, 7), _x(700, L.D, dev, 8)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(a):
+        want = run(x)
+    first = {t.data_ptr(): t.numel() * t.element_size() for t in held().tensors}
+    a.synchronize()
+    b.wait_stream(a)
+    with torch.cuda.stream(b):
+        torch.cuda._sleep(20_000_000)
+        got = run(x)
+        run(longer)                                           # drops the first scratch
+    with torch.cuda.stream(a):
+        other = [torch.empty(n, dtype=torch.uint8, device=dev) for n in first.values()]
+        busy = not b.query()
+        for t in other:
+            t.fill_(255)
+    torch.cuda.synchronize()
+    assert busy, "b was done before a allocated: nothing tested"
+    for t in other:
+        assert all(t.data_ptr() + t.numel() <= p or p + n <= t.data_ptr() for p, n in first.items())
+    _same(got, want)
+
+
 @pytest.mark.parametrize("table", ["k2", "cb"])
 def test_grouped_prompt_refuses_bad_table_entries(dev, ext, table):
     """A width outside the launch's range, or a codebook with no kernel: NaN sums and a status bit, no copy."""

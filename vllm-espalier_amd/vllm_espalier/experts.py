@@ -32,6 +32,7 @@ from pathlib import Path
 import torch
 
 from ._env import env
+from ._streams import hand_out
 
 # Espalier grid code (EspMatrix.cb) -> the kernels' codebook id (exllamav3's: 1 mcg, 3 E2M1, 6 int5, 7 int6)
 KERNEL_CB = {0: 1, 1: 3, 3: 6, 4: 7}
@@ -272,7 +273,7 @@ class Scratch:
             if self.prompt is not None and self.prompt.captured:
                 self.kept.append(self.prompt)
             self.prompt = PrefillScratch(L.E, L.D, L.I, rows, self.slots, self.z.device)
-        return self.prompt.handed_out()
+        return self.prompt
 
     def window(self, R: int):
         """(ids, members [maxu, R]) views for a window of R tokens."""
@@ -451,6 +452,7 @@ class PrefillScratch:
     def __init__(self, E: int, D: int, I: int, rows: int, slots: int, device, window: int = 32):
         self.rows, self.slots, self.E, self.window = rows, slots, E, window
         self.captured = False                            # handed out during a graph capture
+        self.streams: set = set()                        # streams that its buffers are recorded on
         P = rows * slots
         maxu = min(P, E)
         f16, f32, i32 = torch.float16, torch.float32, torch.int32
@@ -464,9 +466,15 @@ class PrefillScratch:
         }
         for name, (shape, dtype, fill) in layout.items():
             setattr(self, name, torch.full(shape, fill, dtype=dtype, device=device))
+        self.tensors = [getattr(self, name) for name in layout]
 
     def handed_out(self) -> PrefillScratch:
-        self.captured |= torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
+        """Note a use on the current stream: a captured one makes whoever replaces this scratch keep it, another holds its
+        memory until that stream is done with it."""
+        if torch.cuda.is_available() and torch.cuda.is_current_stream_capturing():
+            self.captured = True
+        else:
+            hand_out(self.tensors, self.streams, self.z.device)
         return self
 
     def grouping(self, T: int):
@@ -538,6 +546,7 @@ def _prefill(x, pick, wts, L: Layer, s: PrefillScratch, k: int, gate, out, out_s
     slots = k + has_shared
     if T > s.rows or slots != s.slots:
         raise ValueError(f"{T}x{slots} slots but the prefill scratch holds {s.rows}x{s.slots}")
+    s.handed_out()
     P = T * slots
     ids, members = s.grouping(T)
     pick_p, wts_p = s.pick[:P], s.wts[:P]
