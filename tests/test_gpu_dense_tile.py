@@ -191,3 +191,35 @@ def test_tile_rejects_small_scratch(dev, ext):
         ext.dense_tile(x, [m.trellis], [m.suh], [m.svh], [0], y, xh, z, cnt, 2 * m.K, experts.KERNEL_CB[m.cb], 3)
     with pytest.raises(RuntimeError, match="SK at most"):
         ext.dense_tile(x, [m.trellis], [m.suh], [m.svh], [0], y, xh, z, cnt, 2 * m.K, experts.KERNEL_CB[m.cb], 129)
+
+
+def test_outgrown_prompt_scratch_outlives_its_streams(dev, monkeypatch):
+    """The prompt scratch allocated on stream a, used on b and outgrown there while b still has that prompt to run: a's next
+    allocations of the same sizes get other memory, and b's results are right."""
+    for name in ("_PROMPT", "_PROMPT_COUNTERS"):
+        monkeypatch.setattr(D, name, type(D._PROMPT)(getattr(D, name).fill, getattr(D, name).dtype))
+    gen = torch.Generator().manual_seed(21)
+    d = D.Dense([WL.matrix(2048, 512, 4, "int6", gen, dev)])
+    x, longer = (torch.randn((T, 2048), generator=gen).to(torch.bfloat16).to(dev) for T in (140, 900))
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(a):
+        want = d.forward_tile(x)
+    first = [(t.data_ptr(), t.numel() * t.element_size()) for t in D.prompt_scratch(dev, 0, 0, 0)]
+    a.synchronize()
+    b.wait_stream(a)
+    with torch.cuda.stream(b):
+        torch.cuda._sleep(20_000_000)
+        got = d.forward_tile(x)
+        d.forward_tile(longer)                                # drops the first scratch
+    assert [t.data_ptr() for t in D.prompt_scratch(dev, 0, 0, 0)] != [p for p, _ in first]
+    with torch.cuda.stream(a):
+        other = [torch.empty(n, dtype=torch.uint8, device=dev) for _, n in first]
+        busy = not b.query()
+        for t in other:
+            t.fill_(255)
+    torch.cuda.synchronize()
+    assert busy, "b was done before a allocated: nothing tested"
+    for t in other:
+        assert all(t.data_ptr() + t.numel() <= p or p + n <= t.data_ptr() for p, n in first)
+    assert torch.equal(got, want)

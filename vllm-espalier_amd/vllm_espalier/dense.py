@@ -18,6 +18,7 @@ from dataclasses import dataclass
 import torch
 
 from ._env import env
+from ._streams import hand_out
 from .experts import KERNEL_CB, ext
 
 MAX_ROWS = 32
@@ -92,12 +93,14 @@ class _SharedScratch:
     """The split-K partials Z (fp32) and the unfused rotation's rows xh (fp16), one pair a device, shared by every
     layer (layers run one after another). Sizes only grow. A pair that a growth replaces is kept for good only when a
     graph may write to it (it was handed out during a stream capture); otherwise it is dropped, and the caching
-    allocator reuses its memory, so a series of growing prompts outside capture keeps only the current pair."""
+    allocator reuses its memory once every stream that it was handed out on is done with it, so a series of growing
+    prompts outside capture keeps only the current pair."""
 
-    def __init__(self, ones: bool = False):
-        self.ones = ones                     # Z every bit set (the all-ones partials of esp_dense_own)
+    def __init__(self, fill=None, dtype=torch.float32):
+        self.fill, self.dtype = fill, dtype  # Z's 32-bit words to begin with (None: any), and its type
         self.current: dict = {}
         self.captured: set = set()          # devices whose current pair was handed out during a capture
+        self.streams: dict = {}             # device -> streams that its current pair was handed out on
         self.retired: list = []
 
     def reserve(self, device, z_floats: int, xh_halves: int):
@@ -106,24 +109,27 @@ class _SharedScratch:
         if have is not None and have[0].numel() >= z_floats and have[1].numel() >= xh_halves:
             if capturing:
                 self.captured.add(device)
+            else:
+                hand_out(have, self.streams[device], device)
             return have
         if have is not None:
             if device in self.captured:
                 self.retired.append(have)
             z_floats, xh_halves = max(z_floats, have[0].numel()), max(xh_halves, have[1].numel())
         self.captured.discard(device)
-        z = (torch.full((max(z_floats, 1),), -1, dtype=torch.int32, device=device).view(torch.float32) if self.ones
-             else torch.empty(max(z_floats, 1), dtype=torch.float32, device=device))
-        pair = (z,
-                torch.empty(max(xh_halves, 1), dtype=torch.float16, device=device))
+        z = torch.empty(max(z_floats, 1), dtype=torch.int32, device=device)
+        if self.fill is not None:
+            z.fill_(self.fill)
+        pair = (z.view(self.dtype), torch.empty(max(xh_halves, 1), dtype=torch.float16, device=device))
         self.current[device] = pair
+        self.streams[device] = set()
         if capturing:
             self.captured.add(device)
         return pair
 
 
 _SHARED = _SharedScratch()
-_OWN = _SharedScratch(ones=True)
+_OWN = _SharedScratch(fill=-1)               # all-ones partials (esp_dense_own)
 
 
 def scratch(device, z_floats: int, xh_halves: int):
@@ -144,20 +150,13 @@ def polls(M: int, sk: int, w: int) -> bool:
 
 
 _PROMPT = _SharedScratch()
-_PROMPT_COUNTERS: dict = {}
+_PROMPT_COUNTERS = _SharedScratch(fill=0, dtype=torch.int32)
 
 
 def prompt_scratch(device, z_floats: int, xh_halves: int, counters: int):
     """(Z, xh, counters) of the device for prompt launches, grown to at least the given sizes (the counters zero, and
     left zero by every launch)."""
-    was_captured = device in _PROMPT.captured            # before reserve: a growth there resets the mark
-    z, xh = _PROMPT.reserve(device, z_floats, xh_halves)
-    cnt = _PROMPT_COUNTERS.get(device)
-    if cnt is None or cnt.numel() < counters:
-        if cnt is not None and (was_captured or device in _PROMPT.captured):
-            _PROMPT.retired.append((cnt,))
-        cnt = _PROMPT_COUNTERS[device] = torch.zeros(max(counters, 1), dtype=torch.int32, device=device)
-    return z, xh, cnt
+    return *_PROMPT.reserve(device, z_floats, xh_halves), _PROMPT_COUNTERS.reserve(device, counters, 0)[0]
 
 
 def _cu_count(device) -> int:
