@@ -112,12 +112,14 @@ int esp_dense_tile(const void* x, int x_dtype, int64_t x_stride, int64_t T, int6
  * device holds (no reference counterpart): the bits of esp_dense at SK = 1, W = 8, for layers of more blocks than that. x,
  * y (at the matrix's first column) as esp_dense; K a multiple of 256. With norm_w the rows are RMSNorm(x + d1 + d2) *
  * norm_w and the residual goes to h_out, as esp_dense_rmsnorm (M at most 2; d1 / d2 may be null). part fp32 scratch: 256
- * floats a row and workgroup (two a compute unit, at most one a 128-column block), all-ones on entry and left so, as
- * esp_dense_own's partials. A wait past ~20 ms sets ESP_STATUS_WAIT_TIMEOUT. */
+ * floats a row and 32 more for each workgroup (two a compute unit, at most one a 128-column block), all-ones on entry and
+ * left so, as esp_dense_own's partials. A workgroup waits wait_us microseconds (0 to 1000000; 0: it looks once) for the
+ * sums that the one before it hands on, then makes them itself: the same bits, at most a block's work more, and the scratch
+ * all-ones at the end all the same. A negative wait_us makes every workgroup do so (a test of that path). */
 int esp_dense_stream(const void* x, int x_dtype, int64_t x_stride, int64_t M, int64_t K, const void* trellis,
                      const void* suh, const void* svh, int64_t N, void* y, int y_dtype, int64_t y_stride, const void* d1,
                      const void* d2, const void* norm_w, double eps, void* h_out, float* part, int64_t part_numel,
-                     int64_t k2, int64_t cb, void* stream);
+                     int64_t wait_us, int64_t k2, int64_t cb, void* stream);
 
 /* dense over a prompt of any number of rows with every weight decoded once (no reference counterpart): the rows rotated
  * into xh and the weights decoded to fp16 into wf, then a GEMM on those fragments whose sums keep the order of a launch

@@ -137,6 +137,28 @@ def test_stream_equals_one_workgroup_a_block(dev, ext, monkeypatch, K, blocks, b
     assert int(ext.status(True)) == 0
 
 
+@pytest.mark.parametrize("wait", [-1, 0])
+@pytest.mark.parametrize("M", [1, 6])
+@pytest.mark.parametrize("K,blocks,bits,grid", [(256, 600, 2, "mcg"), (2048, 513, 4, "int6"), (1024, 1187, 3, "int5")])
+def test_stream_without_its_predecessors_sums(dev, ext, monkeypatch, K, blocks, bits, grid, M, wait):
+    """Workgroups that give up on their predecessor's sums (all of them; those that come too early) make them themselves: the
+    same bits, and the hand-off buffer all-ones for the launches after, which wait as ever."""
+    gen = torch.Generator(device=dev).manual_seed(K + blocks)
+    d = D.Dense([WL.matrix(K, 128 * blocks, bits, grid, gen, dev)])
+    assert d._streams(M, d.launches[0])
+    monkeypatch.setattr(D, "STREAM", False)
+    xs = [_rows(M, K, torch.bfloat16, dev, M + i) for i in range(4)]
+    want = [d.forward(x) for x in xs]
+    monkeypatch.setattr(D, "STREAM", True)
+    for us in (wait, D.STREAM_WAIT_US, wait, wait):
+        monkeypatch.setattr(D, "STREAM_WAIT_US", us)
+        got = [d.forward(x) for x in xs]
+        torch.cuda.synchronize()
+        assert all(torch.equal(g, w) for g, w in zip(got, want)), us
+        assert bool((d._stream_part(dev).view(torch.int32) == -1).all()), us
+    assert int(ext.status(True)) == 0
+
+
 @pytest.mark.parametrize("M", [1, 2])
 def test_stream_rmsnorm_equals_dense_rmsnorm(dev, monkeypatch, M):
     gen = torch.Generator(device=dev).manual_seed(9)

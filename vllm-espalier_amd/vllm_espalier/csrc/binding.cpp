@@ -364,7 +364,7 @@ void dense_own(const at::Tensor& x, const std::vector<at::Tensor>& T, const std:
 void dense_stream(const at::Tensor& x, const c10::optional<at::Tensor>& d1, const c10::optional<at::Tensor>& d2,
                   const c10::optional<at::Tensor>& norm_w, double eps, const c10::optional<at::Tensor>& h_out,
                   const at::Tensor& T, const at::Tensor& suh, const at::Tensor& svh, int64_t col0, at::Tensor y,
-                  at::Tensor part, int64_t k2, int64_t cb) {
+                  at::Tensor part, int64_t wait_us, int64_t k2, int64_t cb) {
     TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1, "x: CUDA [M, K], unit column stride");
     TORCH_CHECK(y.is_cuda() && y.dim() == 2 && y.stride(1) == 1 && y.size(0) >= x.size(0),
                 "y: CUDA [M, N], unit column stride");
@@ -389,8 +389,8 @@ void dense_stream(const at::Tensor& x, const c10::optional<at::Tensor>& d1, cons
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     call(esp_dense_stream(x.data_ptr(), dtype_code(x), x.stride(0), x.size(0), K, T.data_ptr(), suh.data_ptr(),
                           svh.data_ptr(), N, static_cast<char*>(y.data_ptr()) + col0 * y.element_size(), dtype_code(y),
-                          y.stride(0), ptr(d1), ptr(d2), ptr(norm_w), eps, ptr(h_out), mptr<float>(part), part.numel(), k2,
-                          cb, cur_stream()));
+                          y.stride(0), ptr(d1), ptr(d2), ptr(norm_w), eps, ptr(h_out), mptr<float>(part), part.numel(),
+                          wait_us, k2, cb, cur_stream()));
 }
 
 // The matrices of a prompt launch, checked, as the C entry points take them

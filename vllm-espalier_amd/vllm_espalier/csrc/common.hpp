@@ -365,7 +365,6 @@ int launch_check(const char* what);
 int dense_status(int clear, hipStream_t st, int* out);     // dense_multi.hip: the dense launches' status word
 int tile_status(int clear, hipStream_t st, int* out);      // dense_tile.hip: the prompt launches' status word
 int dense_own_status(int clear, hipStream_t st, int* out); // dense.hip: esp_dense_own's status word
-int dense_stream_status(int clear, hipStream_t st, int* out); // dense_stream.hip: the streamed launches' status word
 int moe_prompt_status(int clear, hipStream_t st, int* out); // moe_prompt.hip: the prompt expert launches' status word
 }  // namespace esp_host
 

@@ -7,11 +7,20 @@
 // workgroup first runs the block that it begins at its share's end and hands its accumulators on (exact fp32, so the next
 // workgroup's MFMAs continue the chain of sums where it broke off), then its whole blocks, and last the block that its
 // predecessor began, whose accumulators are there by then.
+//
+// No result depends on that order in time. A workgroup whose predecessor's sums stay away past a.wait (its XCD held by
+// another stream, a time slice of another process) gives up on them and runs the block from its first stage: the same sums
+// in the same order, at most a block's work again. The buffer is all-ones again when the launch ends, whichever of the two
+// comes last. Wave w of both holds the same KiB of the sums, with a flag word of its own:
+//   the predecessor   stores its KiB, waits until the stores are done, then reads the flag; if the flag is taken (0) it
+//                     puts the all-ones back over the KiB and the flag;
+//   the successor     takes the flag, waits until that store is done, then looks once more: bytes that are there by now it
+//                     puts back to all-ones; if all of them are there, the flag too.
+// Bytes that the successor does not see are stored after the flag was taken, so the predecessor sees the flag taken. Bytes
+// that it sees may be put back twice.
 #include "dense.hpp"
 
 namespace esp {
-
-__device__ int g_stream_status;           // ESP_STATUS_* bits raised by the launches of this file
 
 struct StreamArgs {
     const uint32_t* T;
@@ -22,7 +31,8 @@ struct StreamArgs {
     int x_dtype, x_stride;
     void* y;
     int y_dtype, y_stride;                // y at the matrix's first column
-    float* part;                          // [workgroups][2][M][128], all-ones between launches
+    float* part;                          // [workgroups][2][M][128], then a line of flags a workgroup: all-ones between launches
+    int64_t wait;                         // clock ticks (10 ns) before a workgroup gives up on its predecessor's sums
     int M, K, NB, xs_stride;
     const uint16_t* nh;                   // the rows are RMSNorm(nh + nd1 + nd2) * nw, as esp_dense_rmsnorm's
     const uint16_t* nd1;
@@ -41,8 +51,7 @@ __host__ __device__ constexpr int ds_stage_bytes(int k2) { return DS_STEPS * 2 *
 // whole blocks, 2: the block that its predecessor began
 struct StreamSeq {
     int b, t, left, phase;
-    int b0, nB, bC, tC, nC;
-    const int SS;
+    int b0, nB, bC, tC, nC, SS;
     __device__ __forceinline__ StreamSeq(unsigned g0, unsigned g1, int ss) : SS(ss) {
         const int first = (int)(g0 / (unsigned)ss), last = (int)(g1 / (unsigned)ss), rest = (int)g0 - first * ss;
         b0 = rest ? first + 1 : first;
@@ -89,6 +98,7 @@ __global__ __launch_bounds__(DS_WAVES * 64, 4) void dense_stream_kernel(StreamAr
     constexpr int UPT = (UNITS + DS_WAVES * 64 - 1) / (DS_WAVES * 64), STAGE_WORDS = ds_stage_bytes(K2) / 4;
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float npart[DS_WAVES], ninv[2];
+    __shared__ int late;                                       // the predecessor's sums stay away
     uint32_t* const stage = reinterpret_cast<uint32_t*>(smem);
     uint16_t* const xs = reinterpret_cast<uint16_t*>(smem + 2 * ds_stage_bytes(K2));
     float* const red = reinterpret_cast<float*>(smem + 2 * ds_stage_bytes(K2) + (size_t)a.M * a.xs_stride * 2);
@@ -103,6 +113,7 @@ __global__ __launch_bounds__(DS_WAVES * 64, 4) void dense_stream_kernel(StreamAr
         const int u = (wave + i * DS_WAVES) * 64 + lane, r = u / UPR;
         t_off[i] = r * NTILES * TW + (u - r * UPR) * 4;
     }
+    if (threadIdx.x == 0) late = 0;
     StreamSeq ahead(g0, g1, SS), cur = ahead;
     auto issue = [&](int buf) __attribute__((always_inline)) {
         const uint32_t* src = a.T + ((size_t)ahead.t * 2 * DS_STEPS * NTILES + (size_t)ahead.b * 8) * TW;
@@ -115,7 +126,7 @@ __global__ __launch_bounds__(DS_WAVES * 64, 4) void dense_stream_kernel(StreamAr
         }
         ahead.next();
     };
-    const int n = (int)(g1 - g0);
+    int n = (int)(g1 - g0);
     issue(0);
     // the rows, rotated, in shared memory (dense_program's arithmetic)
     const int chunks = a.K >> 7;
@@ -153,39 +164,72 @@ __global__ __launch_bounds__(DS_WAVES * 64, 4) void dense_stream_kernel(StreamAr
         acc[0][0] = acc[1][0] = f32x4{0.f, 0.f, 0.f, 0.f};
     };
     const DevBuf pb(a.part);
-    const int piece = 2 * M * 128;
-    bool begun = false;                                       // the predecessor's sums are taken over
+    const int piece = 2 * M * 128, mine = (int)threadIdx.x * 4;           // a KiB each of waves 0 .. M - 1
+    const bool carries = wave < M;
+    constexpr uint32_t empty = 0xFFFFFFFFu;
+    const float4 ones = make_float4(__uint_as_float(empty), __uint_as_float(empty), __uint_as_float(empty),
+                                    __uint_as_float(empty));
+    auto landed = [&](const float4& u) __attribute__((always_inline)) {
+        return __float_as_uint(u.x) != empty && __float_as_uint(u.y) != empty && __float_as_uint(u.z) != empty &&
+               __float_as_uint(u.w) != empty;
+    };
+    auto flag = [&](int w) __attribute__((always_inline)) {               // this wave's of workgroup w
+        return reinterpret_cast<int*>(a.part + (size_t)gridDim.x * piece) + (size_t)w * CNT_STRIDE + wave;
+    };
+    bool begun = false, handed = false;                       // the predecessor's sums are taken over; the own ones stored
+    int told = (int)empty;                                    // and the flag read then
     for (int q = 0; q < n; ++q) {
         wait_stage();                                         // the stage landed; every wave is done with the other buffer
         if (q + 1 < n) issue((q + 1) & 1);
+        if (handed) {                                         // the stores are done (wait_stage)
+            handed = false;
+            told = load_dev(flag(wg));
+        }
         if (cur.phase == 2 && !begun) {
             begun = true;
-            const int i = (int)threadIdx.x * 4;
-            if (i < piece) {
-                float* p = a.part + (size_t)(wg - 1) * piece + i;
-                constexpr uint32_t empty = 0xFFFFFFFFu;
+            float* p = a.part + (size_t)(wg - 1) * piece + mine;
+            bool here = true;
+            if (carries) {
                 float4 u = pb.load4(p);
                 const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
-                while (__float_as_uint(u.x) == empty || __float_as_uint(u.y) == empty || __float_as_uint(u.z) == empty ||
-                       __float_as_uint(u.w) == empty) {
+                here = a.wait >= 0 && landed(u);
+                while (!here && (int64_t)(__builtin_amdgcn_s_memrealtime() - t0) < a.wait) {
                     __builtin_amdgcn_s_sleep(1);
-                    if (__builtin_amdgcn_s_memrealtime() - t0 > 2000000ull) {
-                        __hip_atomic_fetch_or(&g_stream_status, ESP_STATUS_WAIT_TIMEOUT, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
-                        break;
-                    }
                     u = pb.load4(p);
+                    here = landed(u);
                 }
-                *reinterpret_cast<float4*>(red + i) = u;
-                const float e = __uint_as_float(empty);
-                pb.store4(p, make_float4(e, e, e, e));
+                if (here) {
+                    *reinterpret_cast<float4*>(red + mine) = u;
+                    pb.store4(p, ones);
+                } else {
+                    late = 1;
+                }
             }
             lds_barrier();
+            if (__builtin_amdgcn_readfirstlane(late)) {
+                if (carries && lane == 0) store_dev(flag(wg - 1), 0);
+                wait_stage();                                 // the flag is taken, and the copies in flight landed
+                if (!here && landed(pb.load4(p))) {
+                    pb.store4(p, ones);
+                    here = true;
+                }
+                const bool all = __ballot(!here) == 0;
+                if (carries && all && lane == 0) store_dev(flag(wg - 1), (int)empty);
+                // the block from its first stage; the stages in shared memory are brought again after the ones before them
+                cur.t = 0;
+                cur.left += cur.tC;
+                n += cur.tC;
+                ahead = cur;
+                issue(q & 1);
+                wait_stage();
+                if (q + 1 < n) issue((q + 1) & 1);
+            } else {
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+                for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (4 * G + r < M) acc[j][0][r] = red[((size_t)kw * M + 4 * G + r) * 128 + 32 * pair + 16 * j + c];
+                    for (int r = 0; r < 4; ++r)
+                        if (4 * G + r < M) acc[j][0][r] = red[((size_t)kw * M + 4 * G + r) * 128 + 32 * pair + 16 * j + c];
+            }
         }
         const uint32_t* bb = stage + (q & 1) * STAGE_WORDS + lane_base;
         // a step's words and rows are read while the step before is decoded
@@ -211,8 +255,9 @@ __global__ __launch_bounds__(DS_WAVES * 64, 4) void dense_stream_kernel(StreamAr
         if (cur.phase == 0) {
             if (cur.left == 1) {                              // the share's last stage of the block: hand the sums on
                 to_red();
-                const int i = (int)threadIdx.x * 4;
-                if (i < piece) pb.store4(a.part + (size_t)wg * piece + i, *reinterpret_cast<const float4*>(red + i));
+                handed = carries;
+                if (carries)
+                    pb.store4(a.part + (size_t)wg * piece + mine, *reinterpret_cast<const float4*>(red + mine));
             }
         } else if (cur.t == SS - 1) {                         // the block's sums are whole: slot 0's plus slot 1's
             to_red();
@@ -229,36 +274,21 @@ __global__ __launch_bounds__(DS_WAVES * 64, 4) void dense_stream_kernel(StreamAr
         }
         cur.next();
     }
+    // a share is at least a block, so a stage followed the one that handed the sums on: the flag was read
+    if (told != (int)empty) {
+        pb.store4(a.part + (size_t)wg * piece + mine, ones);
+        if (lane == 0) store_dev(flag(wg), (int)empty);
+    }
 }
 
 }  // namespace esp
 
 using namespace esp;
 
-namespace esp_host {
-// the streamed dense launches' device status word into *out (ORed), cleared if asked (esp_status)
-int dense_stream_status(int clear, hipStream_t st, int* out) {
-    int v = 0;
-    if (hipMemcpyFromSymbolAsync(&v, HIP_SYMBOL(g_stream_status), sizeof(int), 0, hipMemcpyDeviceToHost, st) !=
-            hipSuccess ||
-        hipStreamSynchronize(st) != hipSuccess)
-        return fail(ESP_ERR_HIP, "status: cannot read the streamed dense launches' status word");
-    *out |= v;
-    if (clear && v) {
-        const int zero = 0;
-        if (hipMemcpyToSymbolAsync(HIP_SYMBOL(g_stream_status), &zero, sizeof(int), 0, hipMemcpyHostToDevice, st) !=
-                hipSuccess ||
-            hipStreamSynchronize(st) != hipSuccess)
-            return fail(ESP_ERR_HIP, "status: cannot clear the streamed dense launches' status word");
-    }
-    return ESP_OK;
-}
-}  // namespace esp_host
-
 extern "C" int esp_dense_stream(const void* x, int x_dtype, int64_t x_stride, int64_t M, int64_t K, const void* trellis,
                                 const void* suh, const void* svh, int64_t N, void* y, int y_dtype, int64_t y_stride,
                                 const void* d1, const void* d2, const void* norm_w, double eps, void* h_out, float* part,
-                                int64_t part_numel, int64_t k2, int64_t cb, void* stream) {
+                                int64_t part_numel, int64_t wait_us, int64_t k2, int64_t cb, void* stream) {
     ESP_REQUIRE(x && trellis && suh && svh && y && part, "dense_stream: null pointer");
     ESP_REQUIRE(M >= 1 && M <= DS_MAX_ROWS, "dense_stream: 1 to 6 rows");
     ESP_REQUIRE(K > 0 && K % (32 * DS_STEPS) == 0 && K <= 65536 && N > 0 && N % 128 == 0 && N < (int64_t(1) << 24) &&
@@ -296,6 +326,7 @@ extern "C" int esp_dense_stream(const void* x, int x_dtype, int64_t x_stride, in
     a.y_dtype = y_dtype;
     a.y_stride = (int)y_stride;
     a.part = part;
+    a.wait = wait_us < 0 ? -1 : wait_us < 1000000 ? wait_us * 100 : 100000000;       // s_memrealtime counts at 100 MHz
     a.M = (int)M;
     a.K = (int)K;
     a.NB = (int)(N / 128);
@@ -314,8 +345,9 @@ extern "C" int esp_dense_stream(const void* x, int x_dtype, int64_t x_stride, in
     const int per_cu = smem <= 80 * 1024 - 512 ? 2 : 1;
     const int wgs = per_cu * cus < a.NB ? per_cu * cus : a.NB;
     ESP_REQUIRE(wgs < 4096, "dense_stream: at most 4095 workgroups");
-    ESP_REQUIRE(part_numel >= (int64_t)wgs * 2 * M * 128, "dense_stream: part needs 256 floats a row and workgroup "
-                                                          "(two a compute unit, at most one a 128-column block)");
+    ESP_REQUIRE(part_numel >= (int64_t)wgs * (2 * M * 128 + CNT_STRIDE),
+                "dense_stream: part needs 256 floats a row and 32 more for each workgroup (two a compute unit, at most one "
+                "a 128-column block)");
     hipStream_t st = (hipStream_t)stream;
     switch (cb * 32 + k2) {
 #define ESP_STREAM_CASE(CB_, K2_)                                                                                       \

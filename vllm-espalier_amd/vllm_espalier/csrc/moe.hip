@@ -2453,7 +2453,6 @@ extern "C" int esp_status(int32_t* status, int clear, void* stream) {
     if (esp_host::tile_status(clear, st, status)) return ESP_ERR_HIP;
     if (esp_host::dense_own_status(clear, st, status)) return ESP_ERR_HIP;
     if (esp_host::moe_prompt_status(clear, st, status)) return ESP_ERR_HIP;
-    if (esp_host::dense_stream_status(clear, st, status)) return ESP_ERR_HIP;
     *status |= v;
     if (clear && v) {
         const int zero = 0;

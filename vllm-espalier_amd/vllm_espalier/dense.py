@@ -83,6 +83,7 @@ OWN = env("ESPALIER_DENSE_OWN", "1") != "0"
 
 
 STREAM_MAX_ROWS = 6          # rows of esp_dense_stream (2 with the norm inside)
+STREAM_WAIT_US = 200         # a workgroup's wait for its predecessor's sums before it makes them itself (the whole launch takes less)
 STREAM_PARTS = 16            # HIP streams of which a layer keeps a hand-off buffer (3 MiB)
 STREAM_SPARES = 4            # captured launches that get one filled beforehand (a fill in the graph: 6 us a replay)
 # wide launches over a few rows run as esp_dense_stream (the same bits); ESPALIER_DENSE_STREAM=0 runs them as esp_dense
@@ -256,7 +257,7 @@ class Dense:
                 smem <= 80 * 1024 - 512)
 
     def _new_parts(self, device, n: int):
-        floats = 2 * _cu_count(device) * 256 * STREAM_MAX_ROWS
+        floats = 2 * _cu_count(device) * (256 * STREAM_MAX_ROWS + COUNTER_STRIDE)
         return torch.full((n, floats), -1, dtype=torch.int32, device=device).view(torch.float32).unbind()
 
     def _stream_part(self, device):
@@ -281,8 +282,8 @@ class Dense:
         """Launch l over the rows of x (at most MAX_ROWS) into its columns of y."""
         if self._streams(x.shape[0], l) and (part := self._stream_part(x.device)) is not None:
             i = l.members[0]
-            ext().dense_stream(x, None, None, None, 0.0, None, codes[i], pre[i], post[i], self.col0[i], y, part, l.k2,
-                               l.cb)
+            ext().dense_stream(x, None, None, None, 0.0, None, codes[i], pre[i], post[i], self.col0[i], y, part,
+                               STREAM_WAIT_US, l.k2, l.cb)
             return
         z, xh = scratch(x.device, 0, 0)
         e = ext()
@@ -395,7 +396,7 @@ class Dense:
         if self._streams(h.shape[0], l) and (part := self._stream_part(h.device)) is not None:
             m = ms[0]
             ext().dense_stream(h, d1, d2, norm_w, eps, h_out, m.trellis, m.suh, m.svh, self.col0[l.members[0]], out,
-                               part, l.k2, l.cb)
+                               part, STREAM_WAIT_US, l.k2, l.cb)
             return out
         z, _ = scratch(h.device, 0, 0)
         ext().dense_rmsnorm(h, d1, d2, norm_w, eps, h_out, [m.trellis for m in ms], [m.suh for m in ms],
