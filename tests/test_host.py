@@ -229,3 +229,27 @@ def test_tile_list_cap_of_taller_tiles(rows):
         used = [c for c in counts if c]
         tiles = sum(-(-c // rows) for c in used)
         assert tiles <= X.tile_list_cap(min(T * k, E), T, T * k, rows)
+
+
+@pytest.mark.parametrize("status", [4, 5, 1])
+def test_check_status_restores_the_hand_off_buffers(monkeypatch, status):
+    """After a wait that gave up, late partials left in the all-ones buffers are gone once check_status has raised; another
+    status leaves the buffers alone."""
+    import types
+    import torch
+    from vllm_espalier import dense as D
+    from vllm_espalier import experts as X
+    monkeypatch.setattr(X, "ext", lambda: types.SimpleNamespace(status=lambda clear: status))
+    monkeypatch.setattr(D, "_OWN", D._SharedScratch(fill=-1))
+    cpu = torch.device("cpu")
+    s = X.Scratch(3, 256, 128, 2, 2, cpu)
+    small = D.own_partials(cpu, 8)
+    D._OWN.captured.add(cpu)                              # a graph holds it: the growth below keeps it
+    bufs = [s.xdc, s.zd, s.logits_n, small, D.own_partials(cpu, 64)]
+    for t in bufs:
+        t.view(-1)[3:5] = 1.0
+    with pytest.raises(RuntimeError):
+        X.check_status()
+    for t in bufs:
+        bits = t.view(torch.int16 if t.dtype == torch.float16 else torch.int32)
+        assert bool((bits == -1).all()) == bool(status & 4)

@@ -144,6 +144,13 @@ def own_partials(device, z_floats: int):
     return _OWN.reserve(device, z_floats, 0)[0]
 
 
+def restore_own_partials() -> None:
+    """Every all-ones partials buffer, those that graphs hold too, all-ones again (after a wait that gave up; nothing may be
+    running)."""
+    for z, _ in [*_OWN.current.values(), *_OWN.retired]:
+        z.view(torch.int32).fill_(-1)
+
+
 def polls(M: int, sk: int, w: int) -> bool:
     """Whether a launch of M rows, sk K splits and w waves takes esp_dense_own's polled hand-off: its last split holds
     one (row, split) partial a 32-lane half."""

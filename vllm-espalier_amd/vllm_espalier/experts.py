@@ -25,6 +25,7 @@ import importlib.machinery
 import importlib.util
 import math
 import os
+import weakref
 from dataclasses import dataclass
 from functools import lru_cache
 from pathlib import Path
@@ -210,12 +211,23 @@ STATUS_BITS = ((1, "a grouped launch met an expert whose (codebook, K2) has no k
                (8, "a tile list held more member tiles than its bound, or a list launch's grid was shorter than it"))
 
 
+WAIT_TIMEOUT = 4
+
+
 def check_status(clear: bool = True) -> None:
     """Raise RuntimeError naming every bit set in the device status word (esp_status: what the kernels met in
     device-resident tables or in-launch hand-offs, which the host cannot see without reading it back), clearing the
     word first if asked. The read synchronises the current stream, so call it outside graph capture: after a prefill,
-    between decode steps, in tests."""
+    between decode steps, in tests. A wait that gave up may leave late partials in a buffer that is all-ones between
+    launches, where a later launch would take them for its own: those buffers are made all-ones again first."""
     v = int(ext().status(clear))
+    if v & WAIT_TIMEOUT:
+        from . import dense
+        if torch.cuda.is_available():
+            torch.cuda.synchronize()                      # the late launches of every stream
+        for s in list(_ALL_SCRATCH):
+            s.restore()
+        dense.restore_own_partials()
     if v:
         raise RuntimeError(f"espalier device status {v:#x}: " + "; ".join(t for b, t in STATUS_BITS if v & b))
 
@@ -225,6 +237,9 @@ def prepare(experts, shared=None, gate_w=None) -> Layer:
     the last table entry, with gate_w its sigmoid-gate weight [D]. Each matrix's suh / svh become rows of the layer's
     stacks."""
     return Layer(experts, shared, gate_w)
+
+
+_ALL_SCRATCH: weakref.WeakSet = weakref.WeakSet()        # every live Scratch
 
 
 class Scratch:
@@ -264,8 +279,14 @@ class Scratch:
         # the logits of esp_route_group_own and esp_route_group_rmsnorm (the shared gate's after each row's E): all-ones
         # between uses
         self.logits_n = torch.full((rows * (E + 1),), -1, dtype=i32, device=device).view(f32)
+        _ALL_SCRATCH.add(self)
         self.prompt: PrefillScratch | None = None        # windows' whole-prompt buffers, grown to the longest prompt
         self.kept: list = []                             # outgrown ones that a captured graph may write to
+
+    def restore(self) -> None:
+        """The buffers that launches leave all-ones, all-ones again (after a wait that gave up; nothing may be running)."""
+        for t, bits in ((self.xdc, torch.int16), (self.zd, torch.int32), (self.logits_n, torch.int32)):
+            t.view(bits).fill_(-1)
 
     def prompt_scratch(self, L: Layer, rows: int) -> PrefillScratch:
         """The PrefillScratch of prompts of up to `rows` tokens that belongs to this scratch."""
