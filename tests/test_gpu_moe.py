@@ -159,6 +159,52 @@ def test_route_rows_equals_windows_and_oracle(dev, ext, R, shared):
     assert np.abs(wts.view(R, slots).cpu().numpy().astype(np.float64) - owts).max() < 1e-6
 
 
+def inexact_rows(R, H, E, dtype, seed):
+    """Rows and router columns whose fp64 sums depend on their order, near midpoints of bf16 values: column e of row r holds
+    b + b 2^-8 (a midpoint) and eight terms of b 2^-54, of which single ones vanish beside b and groups do not, each at its
+    own place; and a shared gate whose sum lies so between two fp32 values. Rows of ordinary data between."""
+    gen = torch.Generator().manual_seed(seed)
+    b, t = (8.0, 2.0 ** -24) if dtype == torch.float16 else (1.0, 2.0 ** -27)        # b * b and t * t = b * b * 2^-54
+    x = torch.randn((R, H), generator=gen)
+    gate = torch.randn((E, H), generator=gen) * 0.02
+    sgate = torch.zeros(H)
+    place = torch.randperm(H, generator=gen)
+    fixed, tiny = place[:2], place[2:]
+    gate[::2] = 0.0
+    sgate[fixed[0]], sgate[fixed[1]] = b, 2.0 ** -10
+    for e in range(0, E, 2):
+        gate[e, fixed[0]], gate[e, fixed[1]] = b, b * 2.0 ** -4
+        gate[e, tiny[8 * e % (H - 16):][:8]] = t
+    for r in range(0, R, 2):
+        x[r] = t
+        x[r, fixed[0]], x[r, fixed[1]] = b, b * 2.0 ** -4
+    sgate[tiny[:12]] = t
+    if dtype == torch.bfloat16:                            # the shared gate alone, at -16, where its sigmoid shows one ulp
+        for r in range(0, R, 4):
+            x[r, fixed[0]], x[r, fixed[1]] = -4.0, -2.0 ** -10
+        sgate[fixed[0]], sgate[fixed[1]] = 4.0, 2.0 ** -10
+        sgate[tiny[:12]] = -2.0 ** -23                     # x 2^-27: the same 2^-54 of the sum
+    return x.to(dtype), gate.to(dtype), sgate.to(dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("R,H,E", [(40, 2048, 256), (7, 256, 33), (50, 2304, 64)])
+def test_route_rows_equals_windows_where_sums_are_inexact(dev, ext, R, H, E, dtype):
+    """route_rows against route_group, bit for bit, where the order of a fp64 sum decides its rounding."""
+    x, gate, sgate = inexact_rows(R, H, E, dtype, R + H)
+    k, sid, slots = 8, E, 9
+    logits = torch.full((R * (E + 1),), float("nan"), dtype=torch.float32, device=dev)
+    pick = torch.full((R * slots,), -7, dtype=torch.int32, device=dev)
+    wts = torch.full((R * slots,), float("nan"), dtype=torch.float32, device=dev)
+    ext.route_rows(x.to(dev), gate.to(dev), sgate.to(dev), k, sid, logits, pick, wts)
+    for r0 in range(0, R, 32):
+        n = min(32, R - r0)
+        lw, pw, ww, *_ = run_route(ext, dev, x[r0:r0 + n].contiguous(), gate, sgate, k, sid)
+        assert torch.equal(lw, logits[r0 * (E + 1):(r0 + n) * (E + 1)]), r0
+        assert torch.equal(pw.reshape(-1), pick[r0 * slots:(r0 + n) * slots]), r0
+        assert torch.equal(ww.reshape(-1), wts[r0 * slots:(r0 + n) * slots]), r0
+
+
 @pytest.mark.parametrize("R", [1, 45])
 def test_route_rows_fp16_strided(dev, ext, R):
     """route_rows with fp16 rows and router weights, the rows a view into wider rows (row stride 2304): the same

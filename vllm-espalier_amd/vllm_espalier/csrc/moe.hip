@@ -1649,13 +1649,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
 // esp_route_rows: a whole prompt's routing in two launches. The router logits on the fp64 matrix cores: a workgroup is
 // RL_WAVES waves on one tile of 16 rows x 16 expert columns, wave w summing the products of K range w with
 // v_mfma_f64_16x16x4f64 (the shared gate's column is the top-k launch's: as a 17th column tile of E = 256 it would take
-// 32 more workgroups than the 512 two a CU hold at 512 rows, a second round for one column). Lane (i, q) of a wave feeds row i's and column i's elements at the same k;
+// 32 more workgroups than the 512 two a CU hold at 512 rows, a second round for one column). Lane (i, q) of a wave feeds
+// row i's and column i's elements at the same k;
 // a step of 32 k gives lane group q the 8 from 8 q (one 16-byte load a lane, 64 contiguous bytes a row), so each MFMA
 // adds 4 products and the steps cover every k once.
-// bf16 x bf16 products are exact in fp64 and so are their sums for ordinary data, so after the one rounding (bf16 for
-// the experts, fp32 for the shared gate) the logits equal route_group's, whose sums run in another order. The waves'
-// partials are added in wave order. Then route_topk_kernel: one wave a row, the shared gate's fp64 dot (as
-// shared_slots_kernel's: the same exact sum) and topk_row.
+// Products of 16-bit values are exact in fp64; a sum of H of them is within H u * H max|x| max|gate| of the exact one in any
+// order (u = 2^-53; so two orders lie within twice that of each other), and the one rounding to bf16 leaves the same bits
+// unless a midpoint of two bf16 values lies between. Where one may (redo), the wave sums the logit again in route_group's
+// order (route_dot), so the logits are route_group's for any input: about one in 10^6 for ordinary data. The waves'
+// partials are added in wave order, four waves on a quarter of the tile each. With the check, both launches at 1531 rows of
+// 2048 and 256 experts take 43.6 us against 40.8 without, 19.2 against 19.2 at 512. Then route_topk_kernel: one wave a row,
+// the shared gate's dot, whose fp32 rounding leaves less room, in route_group's order at once, and topk_row.
 // ------------------------------------------------------------------------------------------------------------------
 constexpr int RL_WAVES = 8;
 constexpr int RL_BATCH = 4;
@@ -1674,11 +1678,50 @@ __device__ __forceinline__ f64x4 route_mfma8(uint4 xv, uint4 gv, f64x4 acc) {
     return acc;
 }
 
+// a wave's dot of one row and one router column (both 8-byte aligned) in route_group's order
+template <int BF16>
+__device__ __forceinline__ double route_dot_wave(const uint16_t* x, const uint16_t* g, int H, int lane) {
+    double acc = 0.0;
+    for (int h0 = 0; h0 < H; h0 += 2048) {
+        uint2 xv[4][2], gv[4][2];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            route_load8(g, h0 + 512 * q + 8 * lane, H, gv[q]);
+            route_load8(x, h0 + 512 * q + 8 * lane, H, xv[q]);
+        }
+        acc = route_dot<BF16>(xv, gv, acc);
+    }
+    return wave_sum_f64_dpp(acc);
+}
+
+// Whether a midpoint of two bf16 values may lie within err >= 0 of d: exactly, where d rounds to a normal bf16 value (whose
+// rounding drops 45 bits of d); else whenever err is not zero. Not for what is no finite number, in any order of its sum.
+__device__ __forceinline__ bool bf16_midpoint_within(double d, double err) {
+    const uint64_t m = __builtin_bit_cast(uint64_t, d) & 0x7FFFFFFFFFFFFFFFull;
+    const int e = (int)(m >> 52);
+    if (e == 0x7FF || !(err > 0.0)) return false;
+    if (e < 1023 - 126 || e >= 1023 + 127) return true;
+    const double off = __builtin_fabs((double)((int64_t)(m & ((1ull << 45) - 1)) - (int64_t)(1ull << 44)));
+    return off * __builtin_bit_cast(double, (uint64_t)(e - 52) << 52) <= err;               // in units of d's last place
+}
+
+// the larger of each half of m and of the absolute 16-bit values in v (their bit patterns order them)
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t max_abs16(uint32_t m, const uint4& v) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        m = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, m),
+                                                                   __builtin_bit_cast(u16x2, w[i] & 0x7FFF7FFFu)));
+    return m;
+}
+
 template <int BF16>
 __global__ __launch_bounds__(RL_WAVES * 64) void route_logits_kernel(const uint16_t* __restrict__ x, int x_stride,
                                                                      const uint16_t* __restrict__ gate, int R, int H,
                                                                      int E, int C, float* __restrict__ logits) {
-    __shared__ double part[RL_WAVES - 1][4][64];
+    __shared__ double part[RL_WAVES][4][64];
+    __shared__ uint16_t xmax[RL_WAVES][16], gmax[RL_WAVES][16];      // each wave's largest |x| a row, |gate| a column
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int i = lane & 15, q = lane >> 4;
     const int r0 = blockIdx.y * 16, c0 = blockIdx.x * 16;
@@ -1686,9 +1729,10 @@ __global__ __launch_bounds__(RL_WAVES * 64) void route_logits_kernel(const uint1
     const int c = c0 + i < E ? c0 + i : E - 1;
     const uint16_t* xr = x + (size_t)r * x_stride;
     const uint16_t* gr = gate + (size_t)c * H;
-    const int kw = H / RL_WAVES;                                // elements of a wave, a multiple of 64
+    const int kw = H / RL_WAVES;                                // elements of a wave, a multiple of 32
     const int kb = wave * kw + 8 * q;                           // a row's 4 lane groups read 64 contiguous bytes
     f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+    uint32_t xm = 0u, gm = 0u;
     int k = 0;
     for (; k + 32 * RL_BATCH <= kw; k += 32 * RL_BATCH) {       // RL_BATCH loads in flight before the first MFMA
         uint4 xv[RL_BATCH], gv[RL_BATCH];
@@ -1698,25 +1742,55 @@ __global__ __launch_bounds__(RL_WAVES * 64) void route_logits_kernel(const uint1
             gv[j] = *reinterpret_cast<const uint4*>(gr + kb + k + 32 * j);
         }
 #pragma unroll
-        for (int j = 0; j < RL_BATCH; ++j) acc = route_mfma8<BF16>(xv[j], gv[j], acc);
+        for (int j = 0; j < RL_BATCH; ++j) {
+            xm = max_abs16(xm, xv[j]);
+            gm = max_abs16(gm, gv[j]);
+            acc = route_mfma8<BF16>(xv[j], gv[j], acc);
+        }
     }
-    for (; k < kw; k += 32)
-        acc = route_mfma8<BF16>(*reinterpret_cast<const uint4*>(xr + kb + k),
-                                *reinterpret_cast<const uint4*>(gr + kb + k), acc);
+    for (; k < kw; k += 32) {
+        const uint4 xv = *reinterpret_cast<const uint4*>(xr + kb + k), gv = *reinterpret_cast<const uint4*>(gr + kb + k);
+        xm = max_abs16(xm, xv);
+        gm = max_abs16(gm, gv);
+        acc = route_mfma8<BF16>(xv, gv, acc);
+    }
+    auto fold = [](uint32_t m) __attribute__((always_inline)) {                // over a lane's halves and the lane groups
+        m = (m >> 16) > (m & 0xFFFFu) ? m >> 16 : m & 0xFFFFu;
+        uint32_t o = __shfl_xor(m, 16, 64);
+        m = o > m ? o : m;
+        o = __shfl_xor(m, 32, 64);
+        return (uint16_t)(o > m ? o : m);
+    };
+    const uint16_t xf = fold(xm), gf = fold(gm);
+    if (q == 0) {
+        xmax[wave][i] = xf;
+        gmax[wave][i] = gf;
+    }
     // lane l holds D[l / 16 + 4 v][l % 16], v = 0..3 (the f64 instruction's layout, unlike the f32 ones' 4 (l / 16) + v)
-    if (wave > 0) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) part[wave - 1][v][lane] = acc[v];
-    }
+    for (int v = 0; v < 4; ++v) part[wave][v][lane] = acc[v];
     __syncthreads();
-    if (wave != 0) return;
+    if (wave >= 4) return;
+    const int v = wave, row = r0 + q + 4 * v, col = c0 + i;     // a wave a quarter of the tile
+    double sum = part[0][v][lane];
+    uint16_t xmx = xmax[0][q + 4 * v], gmx = gmax[0][i];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        double sum = acc[v];
-        for (int w = 1; w < RL_WAVES; ++w) sum += part[w - 1][v][lane];
-        const int row = r0 + q + 4 * v, col = c0 + i;
-        if (row < R && col < E) logits[(size_t)row * C + col] = bf2f(f64_to_bf16(sum));
+    for (int w = 1; w < RL_WAVES; ++w) {
+        sum += part[w][v][lane];
+        xmx = xmax[w][q + 4 * v] > xmx ? xmax[w][q + 4 * v] : xmx;
+        gmx = gmax[w][i] > gmx ? gmax[w][i] : gmx;
     }
+    // 2^-52 between two orders; twice that for the midpoint below a power of two, which lies nearer, and twice again
+    const double err = (double)H * H * 0x1p-50 * bits16_to_f64(gmx, BF16) * bits16_to_f64(xmx, BF16);
+    const bool used = row < R && col < E;
+    uint16_t l = f64_to_bf16(sum);
+    for (uint64_t redo = __ballot(used && bf16_midpoint_within(sum, err)); redo != 0; redo &= redo - 1) {
+        const int at = __builtin_ctzll(redo);                   // wave-uniform: one logit after another, all lanes on it
+        const double s = route_dot_wave<BF16>(x + (size_t)(r0 + (at >> 4) + 4 * v) * x_stride,
+                                              gate + (size_t)(c0 + (at & 15)) * H, H, lane);
+        if (lane == at) l = f64_to_bf16(s);
+    }
+    if (used) logits[(size_t)row * C + col] = bf2f(l);
 }
 
 __global__ __launch_bounds__(256) void route_topk_kernel(float* __restrict__ logits, int R, int E, int k,
@@ -1729,32 +1803,9 @@ __global__ __launch_bounds__(256) void route_topk_kernel(float* __restrict__ log
     const bool has = shared_id >= 0;
     const int C = E + has, slots = k + has;
     float ls = 0.f;
-    if (has) {                                                 // the shared gate's logit: x . sgate, one rounding
-        double acc = 0.0;                                      // 2048 k at a time, all their loads in flight
-        for (int h0 = 0; h0 < H; h0 += 2048) {
-            uint2 xu[8], wu[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int h = h0 + 4 * lane + 256 * j;
-                if (h < H) {
-                    xu[j] = *reinterpret_cast<const uint2*>(x + (size_t)r * x_stride + h);
-                    wu[j] = *reinterpret_cast<const uint2*>(sgate + h);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                if (h0 + 4 * lane + 256 * j >= H) break;
-                const uint16_t xh[4] = {(uint16_t)(xu[j].x & 0xFFFFu), (uint16_t)(xu[j].x >> 16),
-                                        (uint16_t)(xu[j].y & 0xFFFFu), (uint16_t)(xu[j].y >> 16)};
-                const uint16_t wh[4] = {(uint16_t)(wu[j].x & 0xFFFFu), (uint16_t)(wu[j].x >> 16),
-                                        (uint16_t)(wu[j].y & 0xFFFFu), (uint16_t)(wu[j].y >> 16)};
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    acc = __builtin_fma((double)(bf16 ? bf2f(xh[q]) : h2f(xh[q])),
-                                        (double)(bf16 ? bf2f(wh[q]) : h2f(wh[q])), acc);
-            }
-        }
-        ls = (float)wave_sum_f64_dpp(acc);
+    if (has) {                                                 // the shared gate's logit: x . sgate, rounded once
+        const uint16_t* xr = x + (size_t)r * x_stride;
+        ls = (float)(bf16 ? route_dot_wave<1>(xr, sgate, H, lane) : route_dot_wave<0>(xr, sgate, H, lane));
         if (lane == 0) logits[(size_t)r * C + E] = ls;
     }
     int e_mine;
