@@ -74,11 +74,41 @@ def _dense(lib, **over):
     # the kernels move 4 elements of a row and 16-byte trellis units at a time: misaligned operands are refused
     (dict(x=18), "aligned"), (dict(y=20), "aligned"), (dict(x_stride=2050), "aligned"), (dict(t=24), "aligned"),
     (dict(col0=2, y_cols=4096), "multiple of 4"),
+    # the kernels hold row strides in 32 bits
+    (dict(M=2, x_stride=1 << 31), "row stride"), (dict(M=2, y_cols=1 << 31), "row stride"),
 ])
 def test_dense_argument_errors(lib, over, needle):
     rc, msg = _dense(lib, **over)
     assert rc == 1, msg                                  # ESP_ERR_ARG
     assert needle in msg
+
+
+@pytest.mark.parametrize("rows,x_stride,y_stride,rc", [(2, 1 << 31, 2048, 1), (2, 2048, 1 << 31, 1), (1, 1 << 31, 1 << 31, 2)])
+def test_row_strides_past_32_bits(lib, rows, x_stride, y_stride, rc):
+    """The streamed and the prompt launches refuse row strides that their 32-bit ones cannot hold; one row's is not used (the
+    next check, of the codebook, answers)."""
+    P, I64, INT = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int
+    one, nc, c0 = (P * 1)(16), (I64 * 1)(2048), (I64 * 1)(0)
+    f = lib.esp_dense_stream
+    f.restype = INT
+    f.argtypes = [P, INT, I64, I64, I64, P, P, P, I64, P, INT, I64, P, P, P, ctypes.c_double, P, P, I64, I64, I64, I64, P]
+    assert f(16, 1, x_stride, rows, 2048, 16, 16, 16, 2048, 16, 1, y_stride, None, None, None, 0.0, None, 16, 1 << 30, 0, 8, 3,
+             None) == rc
+    assert rc == 2 or "row stride" in lib.esp_last_error().decode()
+    f = lib.esp_dense_prompt
+    f.restype = INT
+    f.argtypes = [P, INT, I64, I64, I64, I64, ctypes.POINTER(P), ctypes.POINTER(P), ctypes.POINTER(P), ctypes.POINTER(I64),
+                  ctypes.POINTER(I64), P, INT, I64, I64, P, I64, P, I64, I64, I64, I64, I64, P]
+    assert f(16, 1, x_stride, rows, 2048, 1, one, one, one, nc, c0, 16, 1, y_stride, 2048, 16, 1 << 30, 16, 1 << 30, 8, 3, 1, 1,
+             None) == rc
+    assert rc == 2 or "row stride" in lib.esp_last_error().decode()
+    f = lib.esp_dense_tile
+    f.restype = INT
+    f.argtypes = [P, INT, I64, I64, I64, I64, ctypes.POINTER(P), ctypes.POINTER(P), ctypes.POINTER(P), ctypes.POINTER(I64),
+                  ctypes.POINTER(I64), P, INT, I64, I64, P, I64, P, I64, P, I64, I64, I64, I64, P]
+    assert f(16, 1, x_stride, rows, 2048, 1, one, one, one, nc, c0, 16, 1, y_stride, 2048, 16, 1 << 30, 16, 1 << 30, 16,
+             1 << 30, 8, 3, 1, None) == rc
+    assert rc == 2 or "row stride" in lib.esp_last_error().decode()
 
 
 def test_dense_unsupported_codebook(lib):

@@ -366,6 +366,10 @@ int dense_status(int clear, hipStream_t st, int* out);     // dense_multi.hip: t
 int tile_status(int clear, hipStream_t st, int* out);      // dense_tile.hip: the prompt launches' status word
 int dense_own_status(int clear, hipStream_t st, int* out); // dense.hip: esp_dense_own's status word
 int moe_prompt_status(int clear, hipStream_t st, int* out); // moe_prompt.hip: the prompt expert launches' status word
+// Whether row strides (elements) fit the kernels' 32-bit ones; one row's stride is not used
+inline bool strides_fit(int64_t rows, int64_t a, int64_t b = 0) {
+    return rows <= 1 || (a < (int64_t(1) << 31) && b < (int64_t(1) << 31));
+}
 }  // namespace esp_host
 
 #define ESP_REQUIRE(cond, ...)                                                                  \

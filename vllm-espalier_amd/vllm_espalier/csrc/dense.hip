@@ -199,7 +199,7 @@ int prepare_dense(const void* x, int x_dtype, int64_t x_stride, int64_t M, int64
                 "K must be a multiple of 128 and SK at most K / 32 (splits of whole 32-k steps)");
     ESP_REQUIRE(x_dtype >= 0 && x_dtype <= 2 && y_dtype >= 0 && y_dtype <= 2, "x / y dtype");
     ESP_REQUIRE(W == 4 || W == 8 || W == 16, "W (waves a workgroup) must be 4, 8 or 16");
-    ESP_REQUIRE(x_stride >= K && y_stride >= y_cols, "x / y row stride");
+    ESP_REQUIRE(x_stride >= K && y_stride >= y_cols && esp_host::strides_fit(M, x_stride, y_stride), "x / y row stride");
     // the kernels move 4 elements of a row at once (8 bytes, 16 for fp32) and trellis tiles 16 bytes at a time
     ESP_REQUIRE(((uintptr_t)x % (x_dtype == ESP_F32 ? 16 : 8)) == 0 && x_stride % 4 == 0 &&
                     ((uintptr_t)y % (y_dtype == ESP_F32 ? 16 : 8)) == 0 && y_stride % 4 == 0,

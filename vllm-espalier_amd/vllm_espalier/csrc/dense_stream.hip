@@ -295,7 +295,8 @@ extern "C" int esp_dense_stream(const void* x, int x_dtype, int64_t x_stride, in
                     K * N <= (int64_t(1) << 33),
                 "dense_stream: K a multiple of 256, N of 128");
     ESP_REQUIRE(x_dtype >= 0 && x_dtype <= 2 && y_dtype >= 0 && y_dtype <= 2, "dense_stream: x / y dtype");
-    ESP_REQUIRE(x_stride >= K && y_stride >= N, "dense_stream: x / y row stride");
+    ESP_REQUIRE(x_stride >= K && y_stride >= N && esp_host::strides_fit(M, x_stride, y_stride),
+                "dense_stream: x / y row stride");
     ESP_REQUIRE(((uintptr_t)x % (x_dtype == ESP_F32 ? 16 : 8)) == 0 && x_stride % 4 == 0 &&
                     ((uintptr_t)y % (y_dtype == ESP_F32 ? 16 : 8)) == 0 && y_stride % 4 == 0,
                 "dense_stream: x / y 8-byte aligned (16 for fp32) with row strides a multiple of 4 elements");

@@ -505,7 +505,8 @@ extern "C" int esp_dense_tile(const void* x, int x_dtype, int64_t x_stride, int6
     ESP_REQUIRE(K > 0 && K % 128 == 0 && SK >= 1 && SK <= K / 32,
                 "dense_tile: K must be a multiple of 128 and SK at most K / 32");
     ESP_REQUIRE(x_dtype >= 0 && x_dtype <= 2 && y_dtype >= 0 && y_dtype <= 2, "dense_tile: x / y dtype");
-    ESP_REQUIRE(x_stride >= K && y_stride >= y_cols, "dense_tile: x / y row stride");
+    ESP_REQUIRE(x_stride >= K && y_stride >= y_cols && esp_host::strides_fit(T, x_stride, y_stride),
+                "dense_tile: x / y row stride");
     ESP_REQUIRE(((uintptr_t)x % (x_dtype == ESP_F32 ? 16 : 8)) == 0 && x_stride % 4 == 0 &&
                     ((uintptr_t)y % (y_dtype == ESP_F32 ? 16 : 8)) == 0 && y_stride % 4 == 0 &&
                     ((uintptr_t)xh & 15) == 0 && ((uintptr_t)Z & 15) == 0,

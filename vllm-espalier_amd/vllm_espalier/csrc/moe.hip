@@ -1882,7 +1882,7 @@ static int route_impl(const void* x, int x_dtype, int64_t x_stride, int64_t R, i
     ESP_REQUIRE(R >= 1 && R * (k + has) <= MAX_PICKS && k + has <= 32, "route_group: window too large");
     ESP_REQUIRE(!has || sgate, "the shared gate weight is needed with a shared slot");
     ESP_REQUIRE(logits_numel >= R * (E + has), "logits scratch too small");
-    ESP_REQUIRE(x_stride >= H && x_stride % 4 == 0, "x row stride");
+    ESP_REQUIRE(x_stride >= H && x_stride % 4 == 0 && esp_host::strides_fit(R, x_stride), "x row stride");
     ESP_REQUIRE(((uintptr_t)x & 7) == 0 && ((uintptr_t)gate & 7) == 0 && (!sgate || ((uintptr_t)sgate & 7) == 0),
                 "route_group: x / gate must be 8-byte aligned");
     ESP_REQUIRE(maxu >= (R * (k + has) < E + has ? R * (k + has) : E + has), "uids too small");
@@ -1953,7 +1953,8 @@ extern "C" int esp_route_rows(const void* x, int x_dtype, int64_t x_stride, int6
     ESP_REQUIRE(!has || sgate, "the shared gate weight is needed with a shared slot");
     ESP_REQUIRE(R >= 1 && (R + 15) / 16 <= 65535, "route_rows: 1 to 1048560 rows");
     ESP_REQUIRE(logits_numel >= R * (E + has), "logits scratch too small");
-    ESP_REQUIRE(x_stride >= H && x_stride % 8 == 0, "route_rows: x row stride a multiple of 8 elements");
+    ESP_REQUIRE(x_stride >= H && x_stride % 8 == 0 && esp_host::strides_fit(R, x_stride),
+                "route_rows: x row stride a multiple of 8 elements");
     ESP_REQUIRE(((uintptr_t)x & 15) == 0 && ((uintptr_t)gate & 15) == 0 && (!sgate || ((uintptr_t)sgate & 15) == 0),
                 "route_rows: x / gate must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
@@ -2017,6 +2018,7 @@ extern "C" int esp_group_shared(const int32_t* pick_in, const float* wts_in, con
     ESP_REQUIRE(!has || (gate_w && x), "a shared slot needs its gate weight");
     ESP_REQUIRE(!has || (x_dtype == ESP_BF16 || x_dtype == ESP_F16), "x: bf16/fp16");
     ESP_REQUIRE(!has || (H % 256 == 0 && x_stride % 4 == 0), "group_shared: H must be a multiple of 256");
+    ESP_REQUIRE(!has || esp_host::strides_fit(R, x_stride), "group_shared: x row stride");
     ESP_REQUIRE(maxu >= (R * slots < E ? R * slots : E), "uids too small");
     ESP_REQUIRE(maxm >= 1, "members too small");
     if (wide_grouping(R, slots, maxm)) {             // the tables, then the grouping
@@ -2044,7 +2046,7 @@ extern "C" int esp_rot_in(const void* x, int x_dtype, int64_t x_stride, const in
     ESP_REQUIRE(x && pick && suh0 && suh1 && out0 && out1, "rot_in: null pointer");
     ESP_REQUIRE(x_dtype == ESP_BF16 || x_dtype == ESP_F16, "x: bf16/fp16");
     ESP_REQUIRE(K % 128 == 0 && K > 0, "K must be a multiple of 128");
-    ESP_REQUIRE(x_stride >= K && x_stride % 4 == 0, "x row stride");
+    ESP_REQUIRE(x_stride >= K && x_stride % 4 == 0 && esp_host::strides_fit(rows, x_stride), "x row stride");
     ESP_REQUIRE((((uintptr_t)x | (uintptr_t)suh0 | (uintptr_t)suh1 | (uintptr_t)out0 | (uintptr_t)out1) & 7) == 0,
                 "rot_in: x, suh and the outputs must be 8-byte aligned");
     ESP_REQUIRE(rows * slots < (int64_t(1) << 31), "rot_in: at most 2^31 - 1 slot rows");
@@ -2168,6 +2170,7 @@ extern "C" int esp_shared_slots(const int32_t* pick_in, const float* wts_in, con
     ESP_REQUIRE(!has || (gate_w && x), "a shared slot needs its gate weight");
     ESP_REQUIRE(!has || (x_dtype == ESP_BF16 || x_dtype == ESP_F16), "x: bf16/fp16");
     ESP_REQUIRE(!has || (H % 256 == 0 && x_stride % 4 == 0), "shared_slots: H must be a multiple of 256");
+    ESP_REQUIRE(!has || esp_host::strides_fit(R, x_stride), "shared_slots: x row stride");
     shared_slots_kernel<<<(unsigned)((R + 3) / 4), 256, 0, (hipStream_t)stream>>>(
         pick_in, wts_in, static_cast<const uint16_t*>(x), (int)x_stride, x_dtype == ESP_BF16,
         static_cast<const uint16_t*>(gate_w), (int)H, (int)shared_id, pick_out, wts_out, (int)R, (int)slots_in);
@@ -2237,6 +2240,7 @@ static int gateup_args(const void* x, int x_dtype, int64_t x_stride, const void*
     ESP_REQUIRE(2 * SK * P * N <= (int64_t(1) << 30), "moe_gateup: the partials must fit in 4 GiB");
     ESP_REQUIRE(maxm >= 1 && maxm <= 32, "at most 32 member rows an expert");
     ESP_REQUIRE(slots >= 1 && slots <= 32, "at most 32 slots a row");
+    ESP_REQUIRE(esp_host::strides_fit(P / slots, x_stride), "x row stride");
     ESP_REQUIRE(lo >= 2 && hi <= 16 && lo <= hi, "K2 range must lie in [2, 16]");
     ESP_REQUIRE(warps == 4 || warps == 8 || warps == 16, "warps (waves a workgroup) must be 4, 8 or 16");
     ESP_REQUIRE(counters_numel >= nexp_max * (N / 128) * CNT_STRIDE, "counters: 32 ints per (expert, 128 columns)");

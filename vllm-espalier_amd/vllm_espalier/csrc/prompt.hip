@@ -352,7 +352,7 @@ extern "C" int esp_dense_prompt(const void* x, int x_dtype, int64_t x_stride, in
     ESP_REQUIRE(K > 0 && K % 128 == 0 && SK >= 1 && (KW == 1 || KW == 2 || KW == 4) && SK * KW <= K / 32,
                 "dense_prompt: K must be a multiple of 128, with a 32-k step for each of SK * KW slots (KW 1, 2 or 4)");
     ESP_REQUIRE(x_dtype >= 0 && x_dtype <= 2 && y_dtype >= 0 && y_dtype <= 2, "dense_prompt: x / y dtype");
-    ESP_REQUIRE(x_stride >= K && x_stride < (int64_t(1) << 31) && y_stride >= y_cols && y_stride < (int64_t(1) << 31),
+    ESP_REQUIRE(x_stride >= K && y_stride >= y_cols && esp_host::strides_fit(T, x_stride, y_stride),
                 "dense_prompt: x / y row stride");
     ESP_REQUIRE(((uintptr_t)x % (x_dtype == ESP_F32 ? 16 : 8)) == 0 && x_stride % 4 == 0 &&
                     ((uintptr_t)y % (y_dtype == ESP_F32 ? 16 : 8)) == 0 && y_stride % 4 == 0 &&
