@@ -85,6 +85,23 @@ def test_windows_given_picks_and_chunks(dev, monkeypatch):
     _same(G.windows(x, pick, wts, L, s, k=k), _by_window(x, pick, wts, L, s, k, None))
 
 
+@pytest.mark.parametrize("rows", [32, 64])
+def test_windows_of_no_finite_values(dev, monkeypatch, rows):
+    """Tokens of infinities, NaN and overflow on the way among ordinary ones: NaN where the window launches give NaN, their
+    bits elsewhere, the other tokens' and the signs of zeros included."""
+    monkeypatch.setattr(G, "tile_rows", lambda *a: rows)
+    L, router, k, s = _layer("wide", dev)
+    x = _x(120, L.D, dev, 15)
+    x[7, 3], x[40, L.D // 2], x[41, L.D - 1] = float("inf"), float("nan"), float("-inf")
+    x[42] = torch.finfo(x.dtype).max
+    x[100] = 0.0
+    want = _by_window(x, None, None, L, s, k, router)
+    for got, w in zip(G.windows(x, None, None, L, s, k=k, gate=router), want):
+        nan = torch.isnan(w)
+        assert bool(nan.any()) and not bool(nan[100].any()) and torch.equal(torch.isnan(got), nan)
+        assert torch.equal(got.view(torch.int16)[~nan], w.view(torch.int16)[~nan])
+
+
 def test_windows_rows_of_8_bytes_alignment(dev):
     """Rows that route_rows does not take (8-byte aligned) still run, as windows."""
     L, router, k, s = _layer("narrow", dev)

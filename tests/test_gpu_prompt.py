@@ -137,6 +137,67 @@ def test_stream_equals_one_workgroup_a_block(dev, ext, monkeypatch, K, blocks, b
     assert int(ext.status(True)) == 0
 
 
+@pytest.mark.parametrize("wait", [-1, 200])
+@pytest.mark.parametrize("M,K,blocks,bits,grid", [(5, 1280, 700, 8, "mcg"), (6, 1280, 257, 8, "mcg"), (6, 4096, 300, 4, "int6"),
+                                                  (6, 8192, 260, 2, "mcg")])
+def test_stream_one_workgroup_a_cu(dev, ext, monkeypatch, M, K, blocks, bits, grid, wait):
+    """esp_dense_stream where its shared memory passes 80 KiB (the package runs esp_dense there): one workgroup a CU."""
+    gen = torch.Generator(device=dev).manual_seed(K + blocks)
+    m = WL.matrix(K, 128 * blocks, bits, grid, gen, dev)
+    d = D.Dense([m])
+    l = d.launches[0]
+    assert not d._streams(M, l)
+    l = D.Launch(l.members, l.k2, l.cb, l.n, 1, 8, 2)             # the plan whose sums the launch keeps
+    d.launches = [l]
+    x = _rows(M, K, torch.bfloat16, dev, M)
+    monkeypatch.setattr(D, "STREAM", False)
+    want = d.forward(x)
+    part, y = d._new_parts(dev, 1)[0], torch.full_like(want, float("nan"))
+    for _ in range(2):
+        ext.dense_stream(x, None, None, None, 0.0, None, m.trellis, m.suh, m.svh, 0, y, part, wait, l.k2, l.cb)
+        assert torch.equal(y, want)
+    assert bool((part.view(torch.int32) == -1).all())
+
+
+def _specials(x):
+    """Rows of infinities, NaN, overflow on the way, the largest and the smallest values among ordinary ones."""
+    T, K = x.shape
+    fin = torch.finfo(x.dtype)
+    x[0, 3], x[1, K // 2], x[2, K - 1] = float("inf"), float("nan"), float("-inf")
+    if T > 5:
+        x[3] = fin.max
+        x[4, ::7], x[4, 1::7] = float("inf"), float("-inf")
+        x[5] = fin.smallest_normal
+    return x
+
+
+def _same_values(got, want):
+    nan = torch.isnan(want)
+    assert torch.equal(torch.isnan(got), nan) and bool(nan.any())
+    assert torch.equal(got[~nan], want[~nan])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("name", ["uneven_slots", "two_steps", "one_step", "nine_blocks", "two_codes"])
+def test_prompt_equals_windows_of_no_finite_values(dev, name, dtype):
+    d = _layer(name, dev)
+    x = _specials(_rows(100, d.K, dtype, dev, 12))
+    _same_values(d.forward_prompt(x), _windows(d, x))
+
+
+@pytest.mark.parametrize("M", [3, 6])
+def test_stream_equals_dense_of_no_finite_values(dev, ext, monkeypatch, M):
+    gen = torch.Generator(device=dev).manual_seed(31)
+    d = D.Dense([WL.matrix(1024, 128 * 700, 4, "int6", gen, dev)])
+    assert d._streams(M, d.launches[0])
+    x = _specials(_rows(M, d.K, torch.bfloat16, dev, 13))
+    monkeypatch.setattr(D, "STREAM", False)
+    want = d.forward(x)
+    monkeypatch.setattr(D, "STREAM", True)
+    _same_values(d.forward(x), want)
+    assert bool((d._stream_part(dev).view(torch.int32) == -1).all()) and int(ext.status(True)) == 0
+
+
 @pytest.mark.parametrize("wait", [-1, 0])
 @pytest.mark.parametrize("M", [1, 6])
 @pytest.mark.parametrize("K,blocks,bits,grid", [(256, 600, 2, "mcg"), (2048, 513, 4, "int6"), (1024, 1187, 3, "int5")])
