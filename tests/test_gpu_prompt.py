@@ -115,6 +115,27 @@ def test_tile_mode_few_rows_of_a_wide_layer(dev):
         assert torch.equal(d.forward_tile(x[:T]), y[:T]), T
 
 
+def test_reserve_prompt_only_for_tile_launches(dev, monkeypatch):
+    """reserve_prompt grows the scratch for launches that run as esp_dense_tile at T rows, and for no others; forward_tile
+    then allocates none."""
+    for name in ("_PROMPT", "_PROMPT_COUNTERS"):
+        monkeypatch.setattr(D, name, type(D._PROMPT)(getattr(D, name).fill, getattr(D, name).dtype))
+    gen = torch.Generator().manual_seed(4)
+    head = D.Dense([WL.matrix(256, 128 * 260, 2, "mcg", gen, dev)])
+    head.reserve_prompt(1)                                     # a decode launch
+    d = _layer("two_steps", dev)
+    d.reserve_prompt(2048)                                     # every weight decoded once
+    assert [how for *_, how in head._tiles(1) + d._tiles(2048)] == ["window", "once"]
+    assert D._PROMPT.current == {} == D._PROMPT_COUNTERS.current
+    d.reserve_prompt(100)
+    assert [how for *_, how in d._tiles(100)] == ["tile"]
+    held = [t.data_ptr() for t in D.prompt_scratch(dev, 0, 0, 0)]
+    x = _rows(100, d.K, torch.bfloat16, dev, 2)
+    want = d.forward_tile(x)
+    assert [t.data_ptr() for t in D.prompt_scratch(dev, 0, 0, 0)] == held
+    assert torch.equal(d.forward_tile(x[:17]), want[:17])
+
+
 @pytest.mark.parametrize("M", [1, 2, 5, 6])
 @pytest.mark.parametrize("K,blocks,bits,grid", [(256, 600, 2, "mcg"), (1024, 260, 4, "int6"), (2048, 517, 6, "mcg"),
                                                 (768, 1187, 3, "int5"), (512, 513, 5, "mcg"), (1280, 700, 8, "mcg")])

@@ -310,17 +310,19 @@ class Dense:
         return (self.K % 128 == 0 and all(m.out_features % 128 == 0 for m in self.mats) and
                 all(self.K * l.n <= PROMPT_WEIGHTS and l.sk * (l.w // 4) <= self.K // 32 for l in self.launches))
 
-    def _tile_is_window(self, T: int, launch) -> bool:
+    def _tile_is_window(self, T: int, launch, sk: int | None = None) -> bool:
         """Whether T rows of a launch in the tile mode run as one decode launch, whose sums are then esp_dense_tile's: no
-        K split and two k slots (the LM head, whose last row a prompt takes: 125 us as a 128-row tile, 72 as a window)."""
-        return T <= MAX_ROWS and launch.sk == 1 == tile_plan(self.K, launch.n) and launch.w == 4 * TILE_SLOTS
+        K split and two k slots (the LM head, whose last row a prompt takes: 125 us as a 128-row tile, 72 as a window).
+        sk: its tile_plan, where the caller has it."""
+        return (T <= MAX_ROWS and launch.sk == 1 and launch.w == 4 * TILE_SLOTS and
+                (tile_plan(self.K, launch.n) if sk is None else sk) == 1)
 
-    def _tile_decodes_once(self, T: int, launch) -> bool:
+    def _tile_decodes_once(self, T: int, launch, sk: int | None = None) -> bool:
         """Whether T rows of a launch in the tile mode run as esp_dense_prompt (the bits of esp_dense_tile, every weight
         decoded once): where esp_dense_tile's grid is past two 8-wave workgroups a CU, so its tiles decode the weights
         again in a second round and its splits' partials follow one another (2048 -> 5120 at 509 / 1024 / 2048 rows: 40
         / 70 / 125 us against 38 / 48 / 76; 4096 -> 2048: 33 / 59 / 105 against 41 / 42 / 57)."""
-        sk = tile_plan(self.K, launch.n)
+        sk = tile_plan(self.K, launch.n) if sk is None else sk
         return (-(-T // TILE_ROWS) * (launch.n // 128) * sk > 512 and self.K * launch.n <= PROMPT_WEIGHTS and
                 sk * TILE_SLOTS <= self.K // 32)
 
@@ -346,14 +348,30 @@ class Dense:
             self._prompt(x, codes, pre, post, y, l, l.sk, l.w // 4)
         return y
 
-    def reserve_prompt(self, T: int) -> None:
-        """Grow the prompt scratch for forward_tile over T rows (done before a graph is captured)."""
-        device = self.mats[0].trellis.device
+    def _tiles(self, T: int) -> list:
+        """(launch, its K splits, how it runs over T rows in the tile mode: "tile", "window" or "once") of every launch."""
+        runs = []
+        for l in self.launches:
+            sk = tile_plan(self.K, l.n)
+            runs.append((l, sk, "window" if self._tile_is_window(T, l, sk) else
+                         "once" if self._tile_decodes_once(T, l, sk) else "tile"))
+        return runs
+
+    def _reserve_tiles(self, T: int, runs, device):
+        """(Z, xh, counters) for the launches of `runs` that run as esp_dense_tile, or None when none does."""
         tiles = -(-T // TILE_ROWS)
-        z = max(tiles * tile_plan(self.K, l.n) * TILE_ROWS * l.n for l in self.launches)
-        xh = max(len(l.members) for l in self.launches) * -(-T // 16) * 16 * self.K
-        cnt = max(tiles * (l.n // 128) * COUNTER_STRIDE for l in self.launches)
-        prompt_scratch(device, z, xh, cnt)
+        z = xh = cnt = 0
+        for l, sk, how in runs:
+            if how == "tile":
+                z = max(z, tiles * sk * TILE_ROWS * l.n)
+                xh = max(xh, len(l.members) * -(-T // 16) * 16 * self.K)
+                cnt = max(cnt, tiles * (l.n // 128) * COUNTER_STRIDE)
+        return prompt_scratch(device, z, xh, cnt) if z else None
+
+    def reserve_prompt(self, T: int) -> None:
+        """Grow the prompt scratch for forward_tile over T rows (done before a graph is captured); launches that run as
+        decode launches or as esp_dense_prompt there need none."""
+        self._reserve_tiles(T, self._tiles(T), self.mats[0].trellis.device)
 
     def forward_tile(self, x, trellis=None, suh=None, svh=None, out=None):
         """x [T, K], any T (a prompt) -> [T, n_out] in x's dtype, each weight decoded once for every 128 rows
@@ -368,21 +386,18 @@ class Dense:
             y[:, self.N:].zero_()
         if x.stride(-1) != 1:
             x = x.contiguous()
-        if not all(self._tile_decodes_once(T, l) or self._tile_is_window(T, l) for l in self.launches):
-            self.reserve_prompt(T)
-        z, xh, cnt = prompt_scratch(x.device, 0, 0, 0)
-        e = ext()
-        for l in self.launches:
-            pick = l.members
-            sk = tile_plan(self.K, l.n)
-            if self._tile_is_window(T, l):
+        runs = self._tiles(T)
+        scratch_tile = self._reserve_tiles(T, runs, x.device)
+        for l, sk, how in runs:
+            if how == "window":
                 self._window(x, codes, pre, post, y, l)
-                continue
-            if self._tile_decodes_once(T, l):
+            elif how == "once":
                 self._prompt(x, codes, pre, post, y, l, sk, TILE_SLOTS)
-                continue
-            e.dense_tile(x, [codes[i] for i in pick], [pre[i] for i in pick], [post[i] for i in pick],
-                         [self.col0[i] for i in pick], y, xh, z, cnt, l.k2, l.cb, sk)
+            else:
+                z, xh, cnt = scratch_tile
+                pick = l.members
+                ext().dense_tile(x, [codes[i] for i in pick], [pre[i] for i in pick], [post[i] for i in pick],
+                                 [self.col0[i] for i in pick], y, xh, z, cnt, l.k2, l.cb, sk)
         return y
 
     def norm_fusable(self, M: int) -> bool:
