@@ -103,13 +103,34 @@ __device__ __forceinline__ void tile_all_arrived(int* counter, int* seen, int to
     __syncthreads();
 }
 
+// xh of esp_dense_tile: a workgroup takes one matrix, one row group of 16 rows and one 128-chunk of K, which fill exactly the
+// 4 (row group, step) A blocks of that chunk: a 32-lane half rotates 2 rows (rows past T are zero) into their fragment
+// places in shared memory, then the 4 KiB go out as one 16-byte store a thread, contiguous in xh. Bound by latency at the
+// sizes that run here, where 4 values a lane beat the prompt launch's 16 (tile_rot_unit): 2048 -> 1024 of two matrices, 512
+// and 1024 rows 6.0 and 6.7 us against 6.6 and 7.4; 33 rows of 4096 3.5 against 4.2.
 __global__ __launch_bounds__(256) void tile_rot_kernel(const void* __restrict__ x, int x_dtype, int x_stride, int T,
-                                                       int K, bool wide, unsigned units, const uint16_t* suh0,
-                                                       const uint16_t* suh1, const uint16_t* suh2, const uint16_t* suh3,
+                                                       int K, const uint16_t* suh0, const uint16_t* suh1,
+                                                       const uint16_t* suh2, const uint16_t* suh3,
                                                        uint16_t* __restrict__ xh, int RG) {
-    const unsigned unit = blockIdx.x * ROT_UNITS + (threadIdx.x >> 3);
-    if (unit < units)
-        tile_rot_unit(unit, x, x_dtype, x_stride, T, K, wide, suh0, suh1, suh2, suh3, xh, RG, [](int st) { return st; });
+    __shared__ __align__(16) uint16_t frag[4 * TILE_FRAG];
+    const int l32 = threadIdx.x & 31, hw = threadIdx.x >> 5;
+    const int nb = K >> 7;
+    const int ch = (int)(blockIdx.x % nb), rg = (int)((blockIdx.x / nb) % RG), s = (int)(blockIdx.x / (nb * RG));
+    const uint16_t* suh = s == 0 ? suh0 : s == 1 ? suh1 : s == 2 ? suh2 : suh3;
+    // the lane's 4 consecutive k (ch * 128 + 4 l32 ...) are 4 consecutive halves of one A fragment lane
+    const int kk = (4 * l32) & 31, kt = kk & 15;
+    const int sl = l32 >> 3;                                  // the step inside the chunk
+    const int G = 2 * (kk >> 4) + ((kt >> 2) & 1), hi = kt >> 3;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int rr = 2 * hw + i, r = rg * 16 + rr;
+        uint2 u = make_uint2(0u, 0u);
+        if (r < T) u = rot128(x, x_dtype, (size_t)r * x_stride + ch * 128, suh + ch * 128, l32);
+        *reinterpret_cast<uint2*>(frag + (sl * 64 + rr + 16 * G) * 8 + 4 * hi) = u;
+    }
+    __syncthreads();
+    uint16_t* dst = xh + (((size_t)s * RG + rg) * (K >> 5) + ch * 4) * TILE_FRAG;
+    reinterpret_cast<uint4*>(dst)[threadIdx.x] = reinterpret_cast<const uint4*>(frag)[threadIdx.x];
 }
 
 // The finisher's rows of one half-wave (rows rbase, rbase + 16, ...): RPB rows at a time with the other splits'
@@ -558,11 +579,10 @@ extern "C" int esp_dense_tile(const void* x, int x_dtype, int64_t x_stride, int6
     const size_t red = (size_t)RED_BYTES + 16;                   // the sums, then the arrival flag
     const size_t smem = stage > red ? stage : red;
     hipStream_t st = (hipStream_t)stream;
-    const long units = (long)n_shards * RG * (K / 128) * 16;     // (matrix, row, 128-chunk)
+    const long units = (long)n_shards * RG * (K / 128);          // (matrix, row group, 128-chunk)
     ESP_REQUIRE(units < (long)1 << 31, "dense_tile: too many rows for one launch");
-    tile_rot_kernel<<<(unsigned)((units + ROT_UNITS - 1) / ROT_UNITS), 256, 0, st>>>(
-        x, x_dtype, (int)x_stride, (int)T, (int)K, rot_wide(x, x_stride, su, (int)n_shards), (unsigned)units, su[0], su[1],
-        su[2], su[3], static_cast<uint16_t*>(xh), (int)RG);
+    tile_rot_kernel<<<(unsigned)units, 256, 0, st>>>(x, x_dtype, (int)x_stride, (int)T, (int)K, su[0], su[1], su[2], su[3],
+                                                     static_cast<uint16_t*>(xh), (int)RG);
     int rc = esp_host::launch_check("dense_tile rotation");
     if (rc) return rc;
     const dim3 grid((unsigned)nbt, (unsigned)SK, (unsigned)tiles);

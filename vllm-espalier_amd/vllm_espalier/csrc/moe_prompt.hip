@@ -5,8 +5,8 @@
 // scaled sums and its readers add them in split order; here the same sums are added in registers as the program passes
 // each split's end (tot), so the launch writes one partial a row, whose bits are those of the splits' sum. One split is
 // esp_grouped's SK = 1.
+#include "../../../include/espalier.h"
 #include "gemm.hpp"
-#include "tile.hpp"
 
 namespace esp {
 
