@@ -253,3 +253,23 @@ def test_check_status_restores_the_hand_off_buffers(monkeypatch, status):
     for t in bufs:
         bits = t.view(torch.int16 if t.dtype == torch.float16 else torch.int32)
         assert bool((bits == -1).all()) == bool(status & 4)
+
+
+@pytest.mark.parametrize("K,N,rows", [(2048, 5120, 97), (4096, 2048, 97), (4096, 256, 97), (8192, 4096, 97), (16384, 256, 97),
+                                      (8192, 512, 97), (4224, 1024, 129), (8192, 2048, 129), (8320, 2048, 161), (12288, 512, 161),
+                                      (16384, 1024, 193), (24576, 1024, 257)])
+def test_prompt_rows_of_long_narrow_layers(monkeypatch, K, N, rows):
+    """Layers of many k and few columns stay windows for longer, and windowed goes by the layer's own number."""
+    import types
+    import torch
+    from vllm_espalier import dense as D
+    from vllm_espalier import ops
+    assert D.prompt_rows(K, N) == rows
+    took = []
+    layer = types.SimpleNamespace(MAX_ROWS=32, n_out=8, prompt_rows=rows, prompts=lambda: True,
+                                  forward=lambda x, *t, out=None: took.append(x.shape[0]),
+                                  forward_prompt=lambda x, *t: took.append(-x.shape[0]))
+    ops.windowed(layer, torch.zeros((rows - 1, 4)))
+    assert sum(took) == rows - 1 and min(took) > 0
+    ops.windowed(layer, torch.zeros((rows, 4)))
+    assert took[-1] == -rows

@@ -69,12 +69,22 @@ def tile_plan(K: int, N: int) -> int:
     return max(1, min(128 // blocks, 8, K // 128))
 
 
+def prompt_rows(K: int, N: int) -> int:
+    """Rows from which a prompt through a K -> N launch runs as esp_dense_prompt (2 launches, each weight decoded once)
+    instead of windows of MAX_ROWS rows, with the same bits. Four windows (97 rows) for most shapes: config 2's four layers
+    together 114 us against 181 at 128 rows, 4096 -> 2048 42 against 45 at 97. But the prompt GEMM walks K in a line, about
+    7 us a 1024 k where its few workgroups do not hide it, while a window's time hardly grows with K (its K splits fill the
+    CUs): past K = 4096 a layer of 512 to 2048 columns takes one window more for each 4096 k (MI355X, windows against prompt:
+    8192 -> 2048 56 / 72 us and 69 / 67 at 97 and 129 rows, 12288 -> 1024 86 / 91 and 103 / 91 at 160 and 192, 16384 -> 1024
+    111 / 114 and 130 / 114 at 192 and 224; 8192 -> 4096 68 / 66 and 16384 -> 256 1.05 at 97)."""
+    if K <= 4096 or N > 2048 or N < 512 or (N < 1024 and K <= 8192):
+        return PROMPT_MIN_ROWS
+    return PROMPT_MIN_ROWS + MAX_ROWS * -(-(K - 4096) // 4096)
+
+
 TILE_ROWS = 128              # rows a prompt-launch workgroup
 TILE_SLOTS = 2               # k slots a workgroup of esp_dense_tile
-# From this many rows a prompt with decode's bits runs as esp_dense_prompt instead of windows of MAX_ROWS rows: 2 launches
-# and each weight decoded once, against a launch a window (config 2's four layers, MI355X: 114 us against 181 us at 128
-# rows; at 96, three windows, a K = 4096 layer alone would lose, 43 us against 39)
-PROMPT_MIN_ROWS = 97
+PROMPT_MIN_ROWS = 97         # rows from which prompt_rows sends a prompt to esp_dense_prompt at the earliest
 PROMPT_ROWS = 4096           # rows one esp_dense_prompt call takes (bounds its scratch)
 PROMPT_WEIGHTS = 1 << 27     # weights a launch decodes whole (2 bytes each)
 # launches whose last K split can poll the others' partials run as esp_dense_own over an all-ones partials buffer (the
@@ -207,6 +217,7 @@ class Dense:
                 members = tuple(run[i:i + MAX_MATRICES])
                 n = sum(self.mats[j].out_features for j in members)
                 self.launches.append(Launch(members, *code, n, *plan(self.K, n, cus)))
+        self.prompt_rows = max(prompt_rows(self.K, l.n) for l in self.launches)
         blocks = max(l.n // 128 for l in self.launches)
         self.counters = torch.zeros(COUNTER_STRIDE * blocks, dtype=torch.int32, device=device)
         scratch(device, max(l.sk * MAX_ROWS * l.n for l in self.launches), 4 * MAX_ROWS * self.K)

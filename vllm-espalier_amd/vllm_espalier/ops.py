@@ -8,7 +8,7 @@ espalier::dense(x, trellis[], suh[], svh[], key) -> [m, n_out] in x's dtype
 
 Rows beyond one launch (prefill) follow ESPALIER_PREFILL_MODE:
     chunk  (default) a row gets exactly its decode bits: the decode kernels over windows of MAX_ROWS rows, or from
-           PROMPT_MIN_ROWS rows the same sums with every weight decoded once (esp_dense_prompt);
+           dense.prompt_rows the same sums with every weight decoded once (esp_dense_prompt);
     gemm   each matrix decoded once (dequant kernel), both Hadamards by the had kernel, and an fp16 matmul
            (hipBLASLt) between them. A layer of HUGE weights or more (the LM head) stays windowed: its decoded weight
            would not fit beside the model;
@@ -23,7 +23,6 @@ import itertools
 import torch
 
 from ._env import env
-from .dense import PROMPT_MIN_ROWS
 
 PREFILL_MODES = ("chunk", "gemm", "tile")
 PREFILL = env("ESPALIER_PREFILL_MODE", "chunk")
@@ -51,7 +50,7 @@ def windowed(layer, x: torch.Tensor, *tensors) -> torch.Tensor:
     step = layer.MAX_ROWS
     if x.shape[0] <= step:
         return layer.forward(x, *tensors)
-    if x.shape[0] >= PROMPT_MIN_ROWS and layer.prompts():
+    if x.shape[0] >= layer.prompt_rows and layer.prompts():
         return layer.forward_prompt(x, *tensors)
     y = x.new_empty((x.shape[0], layer.n_out))
     for r0 in range(0, x.shape[0], step):
