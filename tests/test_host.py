@@ -273,3 +273,22 @@ def test_prompt_rows_of_long_narrow_layers(monkeypatch, K, N, rows):
     assert sum(took) == rows - 1 and min(took) > 0
     ops.windowed(layer, torch.zeros((rows, 4)))
     assert took[-1] == -rows
+
+
+@pytest.mark.parametrize("K,N,grid,bits,T,once", [
+    (2048, 5120, "int6", 4, 513, True), (2048, 5120, "int6", 4, 512, False),                # 600 and 480 workgroups
+    (8192, 2048, "int6", 4, 544, False), (8192, 2048, "int6", 4, 545, True),                # a last tile of 32 rows
+    (1024, 16384, "mcg", 4, 520, False), (1024, 16384, "int5", 4, 520, True), (2048, 4096, "mcg", 3, 520, True),
+    (12288, 4096, "mcg", 4, 768, False), (12288, 4096, "mcg", 4, 900, True), (12288, 4096, "mcg", 8, 640, True),
+    (4096, 24576, "mcg", 4, 640, False), (4096, 24576, "mcg", 4, 700, True), (8192, 2048, "mcg", 2, 576, False),
+    (8192, 2048, "mcg", 2, 700, True), (2048, 1024, "int5", 4, 1024, False), (2048, 1024, "int5", 4, 1025, True)])
+def test_tile_mode_route_by_shape(K, N, grid, bits, T, once):
+    """The line between esp_dense_tile and esp_dense_prompt in the tile mode, either side of it."""
+    import torch
+    from vllm_espalier import dense as D
+    from vllm_espalier import workloads as WL
+    m = WL.matrix(128, 128, bits, grid, torch.Generator().manual_seed(1), torch.device("cpu"))
+    d = D.Dense([m])
+    d.K = K
+    launch = D.Launch((0,), 2 * bits, D.KERNEL_CB[m.cb], N, *D.plan(K, N, 256))
+    assert d._tile_decodes_once(T, launch) is once

@@ -332,10 +332,22 @@ class Dense:
         """Whether T rows of a launch in the tile mode run as esp_dense_prompt (the bits of esp_dense_tile, every weight
         decoded once): where esp_dense_tile's grid is past two 8-wave workgroups a CU, so its tiles decode the weights
         again in a second round and its splits' partials follow one another (2048 -> 5120 at 509 / 1024 / 2048 rows: 40
-        / 70 / 125 us against 38 / 48 / 76; 4096 -> 2048: 33 / 59 / 105 against 41 / 42 / 57)."""
+        / 70 / 125 us against 38 / 48 / 76; 4096 -> 2048: 33 / 59 / 105 against 41 / 42 / 57). The second round has to cost
+        something, so the line lies later (MI355X, tile against prompt, us):
+          a last tile of up to 32 rows costs next to nothing: from K = 4096, and for the mcg weights (cheaper to decode) of
+          large layers, it is not counted (8192 -> 2048 at 520 rows 52 / 60, 12288 -> 4096 of int6 123 / 126);
+          mcg below 8 bits: 800 workgroups from K = 12288 (12288 -> 4096 at 768 / 900 rows 134 / 139 and 165 / 147), 1000
+          from 192 column blocks (4096 -> 24576 at 512 / 700 rows 163 / 168 and 232 / 224), 640 for up to 2048 columns from
+          K = 8192 (8192 -> 2048 of 2 bits at 576 / 700 rows 56 / 61 and 62 / 61)."""
         sk = tile_plan(self.K, launch.n) if sk is None else sk
-        return (-(-T // TILE_ROWS) * (launch.n // 128) * sk > 512 and self.K * launch.n <= PROMPT_WEIGHTS and
-                sk * TILE_SLOTS <= self.K // 32)
+        K, blocks = self.K, launch.n // 128
+        cheap = launch.cb == KERNEL_CB[0] and launch.k2 < 16
+        uncounted = 32 if K >= 4096 or (cheap and K * launch.n >= 1 << 24) else 0
+        limit = 512
+        if cheap:
+            limit = 800 if K >= 12288 else 1000 if blocks >= 192 else 640 if K >= 8192 and blocks <= 16 else 512
+        return (-(-max(T - uncounted, 0) // TILE_ROWS) * blocks * sk > limit and K * launch.n <= PROMPT_WEIGHTS and
+                sk * TILE_SLOTS <= K // 32)
 
     def _prompt(self, x, codes, pre, post, y, launch, sk: int, slots: int) -> None:
         pick = launch.members
