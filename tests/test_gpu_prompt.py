@@ -1,6 +1,8 @@
 """esp_dense_prompt (Dense.forward_prompt, and forward_tile past its rule): every weight decoded once, with the bits of the
 launches whose sums it keeps. No tolerance: the windows (esp_dense) and the tile launch (esp_dense_tile), themselves held
 to the oracle elsewhere, are the reference, bit for bit."""
+import dataclasses
+
 import pytest
 import torch
 
@@ -136,6 +138,15 @@ def test_reserve_prompt_only_for_tile_launches(dev, monkeypatch):
     assert torch.equal(d.forward_tile(x[:17]), want[:17])
 
 
+def _streamed(d):
+    """d with its launch as esp_dense_stream for 1 to 6 rows, whatever the package's rule: any layer at one K split and 8
+    waves (its shares may be one workgroup a CU)."""
+    l = d.launches[0]
+    assert (l.sk, l.w) == (1, 8)
+    d.launches = [dataclasses.replace(l, stream=range(1, D.STREAM_MAX_ROWS + 1))]
+    return d
+
+
 @pytest.mark.parametrize("M", [1, 2, 5, 6])
 @pytest.mark.parametrize("K,blocks,bits,grid", [(256, 600, 2, "mcg"), (1024, 260, 4, "int6"), (2048, 517, 6, "mcg"),
                                                 (768, 1187, 3, "int5"), (512, 513, 5, "mcg"), (1280, 700, 8, "mcg")])
@@ -143,10 +154,7 @@ def test_stream_equals_one_workgroup_a_block(dev, ext, monkeypatch, K, blocks, b
     """esp_dense_stream against esp_dense: shares that end inside blocks, blocks of one stage, as many blocks as workgroups;
     launches in a row, the hand-off buffer left all-ones and no wait timed out."""
     gen = torch.Generator(device=dev).manual_seed(K + blocks)
-    d = D.Dense([WL.matrix(K, 128 * blocks, bits, grid, gen, dev)])
-    l = d.launches[0]
-    if not d._streams(M, l):
-        pytest.skip("the rows do not leave two workgroups a CU")
+    d = _streamed(D.Dense([WL.matrix(K, 128 * blocks, bits, grid, gen, dev)]))
     for dtype in (torch.bfloat16, torch.float16):
         x = _rows(M, K, dtype, dev, M)
         monkeypatch.setattr(D, "STREAM", False)
@@ -226,8 +234,7 @@ def test_stream_without_its_predecessors_sums(dev, ext, monkeypatch, K, blocks, 
     """Workgroups that give up on their predecessor's sums (all of them; those that come too early) make them themselves: the
     same bits, and the hand-off buffer all-ones for the launches after, which wait as ever."""
     gen = torch.Generator(device=dev).manual_seed(K + blocks)
-    d = D.Dense([WL.matrix(K, 128 * blocks, bits, grid, gen, dev)])
-    assert d._streams(M, d.launches[0])
+    d = _streamed(D.Dense([WL.matrix(K, 128 * blocks, bits, grid, gen, dev)]))
     monkeypatch.setattr(D, "STREAM", False)
     xs = [_rows(M, K, torch.bfloat16, dev, M + i) for i in range(4)]
     want = [d.forward(x) for x in xs]
@@ -263,7 +270,7 @@ def test_stream_graph_replay(dev):
     d = D.Dense([WL.matrix(1024, 128 * 700, 4, "mcg", gen, dev)])
     x = _rows(1, d.K, torch.bfloat16, dev, 1)
     want = d.forward(x)
-    calls = D.STREAM_SPARES + 2                                # the last ones fill their buffer in the graph
+    calls = D.STREAM_SPARES + 2                                # the last ones run as esp_dense
     y = torch.empty((calls, *want.shape), dtype=want.dtype, device=dev)
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g):

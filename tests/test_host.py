@@ -292,3 +292,15 @@ def test_tile_mode_route_by_shape(K, N, grid, bits, T, once):
     d.K = K
     launch = D.Launch((0,), 2 * bits, D.KERNEL_CB[m.cb], N, *D.plan(K, N, 256))
     assert d._tile_decodes_once(T, launch) is once
+
+
+@pytest.mark.parametrize("K,blocks,k2,rows", [
+    (2048, 1187, 12, range(1, 7)), (2048, 256, 12, range(0)), (2048, 257, 12, range(1, 7)), (2048, 1000, 4, range(4, 7)),
+    (2048, 1000, 2, range(0)), (2048, 300, 16, range(1, 4)), (4096, 1000, 8, range(1, 6)), (512, 600, 8, range(0)),
+    (512, 1187, 8, range(1, 7)), (768, 500, 6, range(1, 7)), (896, 500, 6, range(0)), (16384, 500, 16, range(0))])
+def test_stream_rows_by_shape(K, blocks, k2, rows):
+    """The rows that a wide layer streams: bits, blocks against CUs, whole stages, shared memory for two workgroups a CU."""
+    from vllm_espalier import dense as D
+    assert list(D.stream_rows(K, 128 * blocks, k2, 1, 1, 8, 256)) == list(rows)
+    for matrices, sk, w in ((2, 1, 8), (1, 2, 8), (1, 1, 4), (1, 1, 16)):
+        assert not D.stream_rows(K, 128 * blocks, k2, matrices, sk, w, 256)

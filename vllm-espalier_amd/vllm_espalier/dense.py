@@ -13,7 +13,7 @@ from __future__ import annotations
 
 import itertools
 import os
-from dataclasses import dataclass
+from dataclasses import dataclass, field
 
 import torch
 
@@ -95,7 +95,7 @@ OWN = env("ESPALIER_DENSE_OWN", "1") != "0"
 STREAM_MAX_ROWS = 6          # rows of esp_dense_stream (2 with the norm inside)
 STREAM_WAIT_US = 200         # a workgroup's wait for its predecessor's sums before it makes them itself (the whole launch takes less)
 STREAM_PARTS = 16            # HIP streams of which a layer keeps a hand-off buffer (3 MiB)
-STREAM_SPARES = 4            # captured launches that get one filled beforehand (a fill in the graph: 6 us a replay)
+STREAM_SPARES = 8            # captured launches that get one; more run as esp_dense (a fill in the graph would take 6 us)
 # wide launches over a few rows run as esp_dense_stream (the same bits); ESPALIER_DENSE_STREAM=0 runs them as esp_dense
 STREAM = env("ESPALIER_DENSE_STREAM", "1") != "0"
 
@@ -194,6 +194,22 @@ class Launch:
     sk: int
     w: int
     pf: int
+    stream: range = field(default=range(0), compare=False)      # rows that run as esp_dense_stream (stream_rows)
+
+
+def stream_rows(K: int, n: int, k2: int, matrices: int, sk: int, w: int, cus: int) -> range:
+    """Rows over which a launch runs as esp_dense_stream: one matrix of more column blocks than CUs in one K split (an LM
+    head), and rows that leave two workgroups a CU. 2048 -> 151936, graph replays: 6 bits (mcg) 73.1 us as a workgroup a block
+    and 66.1 streamed at one row, 76.8 and 67.9 at four; 4 bits (int6) 77.7 and 73.2, 106.9 and 76.4. At 2 bits a block is
+    decoded too soon for the shares to pay below four rows (2048 -> 128000, e2m1, at one and four rows 61 and 63 us, 82 and
+    64), at one bit at none (42 and 45); nor do they in a block of one or two stages, but where the blocks' last round of
+    workgroups is long (512 -> 76800, int6 4 bits: 17.1 and 17.4 us; 512 -> 151936, mcg: 1.04 to 1.12)."""
+    blocks = n // 128
+    if not (matrices == 1 and sk == 1 and w == 4 * TILE_SLOTS and K % 256 == 0 and K * n <= 1 << 33 and n < 1 << 24 and
+            blocks > cus and k2 >= 4 and (K >= 768 or blocks > 4 * cus)):
+        return range(0)
+    fit = (80 * 1024 - 512 - 4096 * k2) // (2 * K + 16 + 1024)
+    return range(4 if k2 == 4 else 1, min(fit, STREAM_MAX_ROWS) + 1)
 
 
 class Dense:
@@ -209,14 +225,14 @@ class Dense:
         self.col0, self.N = offsets[:-1], offsets[-1]
         self.n_out = n_out or self.N
         device = self.mats[0].trellis.device
-        cus = _cu_count(device)
+        self.cus = cus = _cu_count(device)
         self.launches = []
         for code, run in itertools.groupby(range(len(self.mats)), key=self._code):
             run = list(run)
             for i in range(0, len(run), MAX_MATRICES):
                 members = tuple(run[i:i + MAX_MATRICES])
                 n = sum(self.mats[j].out_features for j in members)
-                self.launches.append(Launch(members, *code, n, *plan(self.K, n, cus)))
+                self.launches.append(self._launch(members, *code, n, *plan(self.K, n, cus)))
         self.prompt_rows = max(prompt_rows(self.K, l.n) for l in self.launches)
         blocks = max(l.n // 128 for l in self.launches)
         self.counters = torch.zeros(COUNTER_STRIDE * blocks, dtype=torch.int32, device=device)
@@ -224,8 +240,11 @@ class Dense:
         own_partials(device, max(l.sk * 2 * l.w // max(l.sk - 1, 1) * l.n for l in self.launches))
         # esp_dense_stream's hand-off buffers: a HIP stream's own, spare ones for captured launches, and those in graphs
         self._stream_parts, self._stream_graphs = {}, []
-        streams = any(self._streams(1, l) for l in self.launches)
+        streams = any(l.stream for l in self.launches)
         self._stream_spare = list(self._new_parts(device, STREAM_SPARES)) if streams else []
+
+    def _launch(self, members, k2, cb, n, sk, w, pf) -> Launch:
+        return Launch(members, k2, cb, n, sk, w, pf, stream_rows(self.K, n, k2, len(members), sk, w, self.cus))
 
     def _code(self, i: int) -> tuple[int, int]:
         m = self.mats[i]
@@ -246,7 +265,7 @@ class Dense:
         """Replace the launches' plans (the scratch must already be large enough for them)."""
         if len(plans) != len(self.launches):
             raise ValueError(f"{len(plans)} plans for {len(self.launches)} launches")
-        self.launches = [Launch(l.members, l.k2, l.cb, l.n, *p) for l, p in zip(self.launches, plans)]
+        self.launches = [self._launch(l.members, l.k2, l.cb, l.n, *p) for l, p in zip(self.launches, plans)]
 
     def forward(self, x, trellis=None, suh=None, svh=None, out=None):
         """x [M, K] (M <= MAX_ROWS) -> [M, n_out] in x's dtype. trellis / suh / svh: lists that replace the matrices'
@@ -264,15 +283,8 @@ class Dense:
         return y
 
     def _streams(self, M: int, l) -> bool:
-        """Whether launch l over M rows runs as esp_dense_stream (its plan's bits): one matrix of more column blocks than
-        CUs in one K split (an LM head), and rows that leave two workgroups a CU. 2048 -> 151936, graph replays: 6 bits
-        (mcg) 73.1 us as a workgroup a block and 66.1 streamed at one row, 76.8 and 67.9 at four; 4 bits (int6) 77.7 and
-        73.2, 106.9 and 76.4."""
-        blocks = l.n // 128
-        smem = 4096 * l.k2 + M * (2 * self.K + 16 + 1024)
-        return (STREAM and 1 <= M <= STREAM_MAX_ROWS and len(l.members) == 1 and l.sk == 1 and l.w == 4 * TILE_SLOTS and
-                self.K % 256 == 0 and self.K * l.n <= 1 << 33 and l.n < 1 << 24 and blocks > 256 and
-                smem <= 80 * 1024 - 512)
+        """Whether launch l over M rows runs as esp_dense_stream (its plan's bits)."""
+        return STREAM and M in l.stream
 
     def _new_parts(self, device, n: int):
         floats = 2 * _cu_count(device) * (256 * STREAM_MAX_ROWS + COUNTER_STRIDE)
@@ -281,13 +293,13 @@ class Dense:
     def _stream_part(self, device):
         """The all-ones hand-off buffer for an esp_dense_stream launch on the current HIP stream, left all-ones by every
         launch: launches on one stream run one after another, and no two streams share one. A captured launch has one of
-        its own, since a graph replays on any stream: a spare one, kept with the layer, or one filled in the graph. None
-        past STREAM_PARTS streams."""
+        its own, since a graph replays on any stream, kept with the layer. None past STREAM_PARTS streams or STREAM_SPARES
+        captured launches."""
         if torch.cuda.is_current_stream_capturing():
             try:
                 part = self._stream_spare.pop()
             except IndexError:
-                return self._new_parts(device, 1)[0]
+                return None
             self._stream_graphs.append(part)
             return part
         key = torch.cuda.current_stream(device).cuda_stream
@@ -298,7 +310,7 @@ class Dense:
 
     def _window(self, x, codes, pre, post, y, l) -> None:
         """Launch l over the rows of x (at most MAX_ROWS) into its columns of y."""
-        if self._streams(x.shape[0], l) and (part := self._stream_part(x.device)) is not None:
+        if x.shape[0] in l.stream and STREAM and (part := self._stream_part(x.device)) is not None:
             i = l.members[0]
             ext().dense_stream(x, None, None, None, 0.0, None, codes[i], pre[i], post[i], self.col0[i], y, part,
                                STREAM_WAIT_US, l.k2, l.cb)
