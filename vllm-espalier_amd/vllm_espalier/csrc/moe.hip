@@ -1658,34 +1658,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
 // unless a midpoint of two bf16 values lies between. Where one may (redo), the wave sums the logit again in route_group's
 // order (route_dot), so the logits are route_group's for any input: about one in 10^6 for ordinary data. The waves'
 // partials are added in wave order, four waves on a quarter of the tile each. With the check, both launches at 1531 rows of
-// 2048 and 256 experts take 43.6 us against 40.8 without, 19.2 against 19.2 at 512. Then route_topk_kernel: one wave a row,
-// the shared gate's dot, whose fp32 rounding leaves less room, in route_group's order at once, and topk_row.
+// 2048 and 256 experts take 42.0 us against 40.9 without, 19.0 against 19.4 at 512 (eight waves a SIMD: 43.5 at the five that
+// the registers of its loads would leave otherwise). Then route_topk_kernel: one wave a row, the shared gate's dot, whose
+// fp32 rounding leaves less room, in route_group's order at once, and topk_row.
 // ------------------------------------------------------------------------------------------------------------------
 constexpr int RL_WAVES = 8;
 constexpr int RL_BATCH = 4;
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-// 8 consecutive k of one row (xv) and one router column (gv): 8 MFMAs, in k order
+// 8 consecutive k of one row (xv) and one router column (gv): 8 MFMAs, in k order; the largest |x| and |gate| so far
 template <int BF16>
-__device__ __forceinline__ f64x4 route_mfma8(uint4 xv, uint4 gv, f64x4 acc) {
+__device__ __forceinline__ f64x4 route_mfma8(uint4 xv, uint4 gv, f64x4 acc, float& xm, float& gm) {
     const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w}, gw[4] = {gv.x, gv.y, gv.z, gv.w};
+    auto f32 = [](uint32_t h) __attribute__((always_inline)) { return BF16 ? bf2f((uint16_t)h) : h2f((uint16_t)h); };
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        const uint32_t xh = (t & 1) ? xw[t >> 1] >> 16 : xw[t >> 1] & 0xFFFFu;
-        const uint32_t gh = (t & 1) ? gw[t >> 1] >> 16 : gw[t >> 1] & 0xFFFFu;
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(bits16_to_f64(xh, BF16), bits16_to_f64(gh, BF16), acc, 0, 0, 0);
+    for (int t = 0; t < 4; ++t) {
+        const float x0 = f32(xw[t] & 0xFFFFu), x1 = f32(xw[t] >> 16), g0 = f32(gw[t] & 0xFFFFu), g1 = f32(gw[t] >> 16);
+        xm = __builtin_fmaxf(__builtin_fmaxf(xm, __builtin_fabsf(x0)), __builtin_fabsf(x1));
+        gm = __builtin_fmaxf(__builtin_fmaxf(gm, __builtin_fabsf(g0)), __builtin_fabsf(g1));
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x0, (double)g0, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x1, (double)g1, acc, 0, 0, 0);
     }
     return acc;
 }
 
-// a wave's dot of one row and one router column (both 8-byte aligned) in route_group's order
-template <int BF16>
+// a wave's dot of one row and one router column (both 8-byte aligned) in route_group's order, with AHEAD chunks of 8 k a lane
+// in flight (4, or 1 for few registers)
+template <int BF16, int AHEAD>
 __device__ __forceinline__ double route_dot_wave(const uint16_t* x, const uint16_t* g, int H, int lane) {
     double acc = 0.0;
-    for (int h0 = 0; h0 < H; h0 += 2048) {
-        uint2 xv[4][2], gv[4][2];
+#pragma unroll 1
+    for (int h0 = 0; h0 < H; h0 += 512 * AHEAD) {
+        uint2 xv[AHEAD][2], gv[AHEAD][2];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < AHEAD; ++q) {
             route_load8(g, h0 + 512 * q + 8 * lane, H, gv[q]);
             route_load8(x, h0 + 512 * q + 8 * lane, H, xv[q]);
         }
@@ -1705,23 +1711,12 @@ __device__ __forceinline__ bool bf16_midpoint_within(double d, double err) {
     return off * __builtin_bit_cast(double, (uint64_t)(e - 52) << 52) <= err;               // in units of d's last place
 }
 
-// the larger of each half of m and of the absolute 16-bit values in v (their bit patterns order them)
-typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t max_abs16(uint32_t m, const uint4& v) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        m = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, m),
-                                                                   __builtin_bit_cast(u16x2, w[i] & 0x7FFF7FFFu)));
-    return m;
-}
-
 template <int BF16>
-__global__ __launch_bounds__(RL_WAVES * 64) void route_logits_kernel(const uint16_t* __restrict__ x, int x_stride,
-                                                                     const uint16_t* __restrict__ gate, int R, int H,
-                                                                     int E, int C, float* __restrict__ logits) {
+__global__ __launch_bounds__(RL_WAVES * 64) __attribute__((amdgpu_waves_per_eu(8))) void route_logits_kernel(
+    const uint16_t* __restrict__ x, int x_stride, const uint16_t* __restrict__ gate, int R, int H, int E, int C,
+    float* __restrict__ logits) {
     __shared__ double part[RL_WAVES][4][64];
-    __shared__ uint16_t xmax[RL_WAVES][16], gmax[RL_WAVES][16];      // each wave's largest |x| a row, |gate| a column
+    __shared__ float xmax[RL_WAVES][16], gmax[RL_WAVES][16];      // each wave's largest |x| a row, |gate| a column
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int i = lane & 15, q = lane >> 4;
     const int r0 = blockIdx.y * 16, c0 = blockIdx.x * 16;
@@ -1732,7 +1727,7 @@ __global__ __launch_bounds__(RL_WAVES * 64) void route_logits_kernel(const uint1
     const int kw = H / RL_WAVES;                                // elements of a wave, a multiple of 32
     const int kb = wave * kw + 8 * q;                           // a row's 4 lane groups read 64 contiguous bytes
     f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-    uint32_t xm = 0u, gm = 0u;
+    float xm = 0.f, gm = 0.f;
     int k = 0;
     for (; k + 32 * RL_BATCH <= kw; k += 32 * RL_BATCH) {       // RL_BATCH loads in flight before the first MFMA
         uint4 xv[RL_BATCH], gv[RL_BATCH];
@@ -1742,29 +1737,20 @@ __global__ __launch_bounds__(RL_WAVES * 64) void route_logits_kernel(const uint1
             gv[j] = *reinterpret_cast<const uint4*>(gr + kb + k + 32 * j);
         }
 #pragma unroll
-        for (int j = 0; j < RL_BATCH; ++j) {
-            xm = max_abs16(xm, xv[j]);
-            gm = max_abs16(gm, gv[j]);
-            acc = route_mfma8<BF16>(xv[j], gv[j], acc);
-        }
+        for (int j = 0; j < RL_BATCH; ++j) acc = route_mfma8<BF16>(xv[j], gv[j], acc, xm, gm);
     }
-    for (; k < kw; k += 32) {
-        const uint4 xv = *reinterpret_cast<const uint4*>(xr + kb + k), gv = *reinterpret_cast<const uint4*>(gr + kb + k);
-        xm = max_abs16(xm, xv);
-        gm = max_abs16(gm, gv);
-        acc = route_mfma8<BF16>(xv, gv, acc);
-    }
-    auto fold = [](uint32_t m) __attribute__((always_inline)) {                // over a lane's halves and the lane groups
-        m = (m >> 16) > (m & 0xFFFFu) ? m >> 16 : m & 0xFFFFu;
-        uint32_t o = __shfl_xor(m, 16, 64);
-        m = o > m ? o : m;
-        o = __shfl_xor(m, 32, 64);
-        return (uint16_t)(o > m ? o : m);
+    for (; k < kw; k += 32)
+        acc = route_mfma8<BF16>(*reinterpret_cast<const uint4*>(xr + kb + k),
+                                *reinterpret_cast<const uint4*>(gr + kb + k), acc, xm, gm);
+    auto fold = [](float m) __attribute__((always_inline)) {                   // over the lane groups
+        m = __builtin_fmaxf(m, __shfl_xor(m, 16, 64));
+        return __builtin_fmaxf(m, __shfl_xor(m, 32, 64));
     };
-    const uint16_t xf = fold(xm), gf = fold(gm);
+    xm = fold(xm);
+    gm = fold(gm);
     if (q == 0) {
-        xmax[wave][i] = xf;
-        gmax[wave][i] = gf;
+        xmax[wave][i] = xm;
+        gmax[wave][i] = gm;
     }
     // lane l holds D[l / 16 + 4 v][l % 16], v = 0..3 (the f64 instruction's layout, unlike the f32 ones' 4 (l / 16) + v)
 #pragma unroll
@@ -1773,21 +1759,21 @@ __global__ __launch_bounds__(RL_WAVES * 64) void route_logits_kernel(const uint1
     if (wave >= 4) return;
     const int v = wave, row = r0 + q + 4 * v, col = c0 + i;     // a wave a quarter of the tile
     double sum = part[0][v][lane];
-    uint16_t xmx = xmax[0][q + 4 * v], gmx = gmax[0][i];
+    float xmx = xmax[0][q + 4 * v], gmx = gmax[0][i];
 #pragma unroll
     for (int w = 1; w < RL_WAVES; ++w) {
         sum += part[w][v][lane];
-        xmx = xmax[w][q + 4 * v] > xmx ? xmax[w][q + 4 * v] : xmx;
-        gmx = gmax[w][i] > gmx ? gmax[w][i] : gmx;
+        xmx = __builtin_fmaxf(xmx, xmax[w][q + 4 * v]);
+        gmx = __builtin_fmaxf(gmx, gmax[w][i]);
     }
     // 2^-52 between two orders; twice that for the midpoint below a power of two, which lies nearer, and twice again
-    const double err = (double)H * H * 0x1p-50 * bits16_to_f64(gmx, BF16) * bits16_to_f64(xmx, BF16);
+    const double err = (double)H * H * 0x1p-50 * (double)gmx * (double)xmx;
     const bool used = row < R && col < E;
     uint16_t l = f64_to_bf16(sum);
     for (uint64_t redo = __ballot(used && bf16_midpoint_within(sum, err)); redo != 0; redo &= redo - 1) {
         const int at = __builtin_ctzll(redo);                   // wave-uniform: one logit after another, all lanes on it
-        const double s = route_dot_wave<BF16>(x + (size_t)(r0 + (at >> 4) + 4 * v) * x_stride,
-                                              gate + (size_t)(c0 + (at & 15)) * H, H, lane);
+        const double s = route_dot_wave<BF16, 1>(x + (size_t)(r0 + (at >> 4) + 4 * v) * x_stride,
+                                                 gate + (size_t)(c0 + (at & 15)) * H, H, lane);
         if (lane == at) l = f64_to_bf16(s);
     }
     if (used) logits[(size_t)row * C + col] = bf2f(l);
@@ -1805,7 +1791,7 @@ __global__ __launch_bounds__(256) void route_topk_kernel(float* __restrict__ log
     float ls = 0.f;
     if (has) {                                                 // the shared gate's logit: x . sgate, rounded once
         const uint16_t* xr = x + (size_t)r * x_stride;
-        ls = (float)(bf16 ? route_dot_wave<1>(xr, sgate, H, lane) : route_dot_wave<0>(xr, sgate, H, lane));
+        ls = (float)(bf16 ? route_dot_wave<1, 4>(xr, sgate, H, lane) : route_dot_wave<0, 4>(xr, sgate, H, lane));
         if (lane == 0) logits[(size_t)r * C + E] = ls;
     }
     int e_mine;

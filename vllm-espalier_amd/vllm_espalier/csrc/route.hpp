@@ -247,11 +247,11 @@ __device__ __forceinline__ void route_load8(const uint16_t* p, int h, int H, uin
     }
 }
 
-// a lane's share of a logit: its 4 chunks of 8 (x, gate) pairs, exact fp64 products added to acc in order
-template <int BF16>
-__device__ __forceinline__ double route_dot(const uint2 (&xv)[4][2], const uint2 (&gv)[4][2], double acc) {
+// a lane's share of a logit: its N chunks of 8 (x, gate) pairs, exact fp64 products added to acc in order
+template <int BF16, int N>
+__device__ __forceinline__ double route_dot(const uint2 (&xv)[N][2], const uint2 (&gv)[N][2], double acc) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < N; ++q) {
         const uint32_t gw[4] = {gv[q][0].x, gv[q][0].y, gv[q][1].x, gv[q][1].y};
         const uint32_t xw[4] = {xv[q][0].x, xv[q][0].y, xv[q][1].x, xv[q][1].y};
 #pragma unroll
