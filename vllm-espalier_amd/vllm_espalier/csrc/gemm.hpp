@@ -162,13 +162,13 @@ __device__ __forceinline__ void block_gemm(const uint32_t* __restrict__ T, int N
             f16x8 av[MG];
 #pragma unroll
             for (int g = 0; g < MG; ++g) aload(g, k0 + 32 * (first + st), av[g]);
+            f16x8 b[2];
+            decode_b2<CB, K2>(w, lp, b);
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const f16x8 b = decode_b<CB, K2>(w[j], lp);
+            for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int g = 0; g < MG; ++g)
-                    acc[j][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[g], b, acc[j][g], 0, 0, 0);
-            }
+                    acc[j][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[g], b[j], acc[j][g], 0, 0, 0);
         }
     }
 }
