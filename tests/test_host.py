@@ -304,3 +304,28 @@ def test_stream_rows_by_shape(K, blocks, k2, rows):
     assert list(D.stream_rows(K, 128 * blocks, k2, 1, 1, 8, 256)) == list(rows)
     for matrices, sk, w in ((2, 1, 8), (1, 2, 8), (1, 1, 4), (1, 1, 16)):
         assert not D.stream_rows(K, 128 * blocks, k2, matrices, sk, w, 256)
+
+
+@pytest.mark.parametrize("E,D,I,slots,most,rows", [
+    (257, 2048, 512, 9, 8192, 4064), (257, 2048, 512, 9, 2048, 2048), (17, 2048, 512, 9, 8192, 8192), (4096, 256, 128, 3, 8192, 256),
+    (64, 16384, 512, 32, 8192, 4095), (8, 8192, 16384, 32, 8192, 4095), (8, 8192, 512, 32, 8192, 8191)])
+def test_pass_rows_bounds_a_whole_prompt_pass(E, D, I, slots, most, rows):
+    """A pass's member table holds at most a million entries and its slot rows are indexed in 31 bits; the scratch for a longer
+    prompt is that of one pass."""
+    import types
+    import torch
+    from vllm_espalier import experts as X
+    L = types.SimpleNamespace(E=E, D=D, I=I)
+    assert X.pass_rows(L, slots, most) == rows
+    assert rows * slots * max(D, I) < 2 ** 31 and (rows <= 32 or E * rows <= X.MEMBER_TABLE)
+
+
+def test_prefill_scratch_holds_one_pass(monkeypatch):
+    import types
+    import torch
+    from vllm_espalier import experts as X
+    monkeypatch.setattr(X, "_PREFILL", {})
+    L = types.SimpleNamespace(E=4096, D=256, I=128)
+    s = X.prefill_scratch(L, 100_000, 3, torch.device("cpu"))
+    assert s.rows == X.pass_rows(L, 3, X.PREFILL_MAX_ROWS) == 256
+    assert X.prefill_scratch(L, 200, 3, torch.device("cpu")) is s

@@ -427,9 +427,13 @@ def routed2(x: torch.Tensor, pick: torch.Tensor | None, wts: torch.Tensor | None
 WINDOWS_PROMPT_ROWS = 2048     # tokens of one whole-prompt pass of windows (bounds its scratch)
 
 
-def _listed_rows(L: Layer) -> int:
-    """Tokens whose (expert, 32-token tile) pairs a tile list holds."""
-    return max(TILE_LIST_PAIRS // L.E, 1) * 32
+MEMBER_TABLE = 1 << 20         # entries (4 MiB) of a pass's member table, a row an expert slot
+
+
+def pass_rows(L: Layer, slots: int, most: int) -> int:
+    """Tokens of one whole-prompt pass, at most `most`: the member table bounded, in whole tiles of 32, and a pass's slot rows
+    within the 31 bits by which the expert launches index them."""
+    return min(most, max(MEMBER_TABLE // L.E // 32, 1) * 32, max((2 ** 31 - 1) // (slots * max(L.D, L.I)), 1))
 
 
 def _whole_prompt(x: torch.Tensor, L: Layer, gate: torch.Tensor | None) -> bool:
@@ -449,7 +453,7 @@ def windows(x: torch.Tensor, pick: torch.Tensor | None, wts: torch.Tensor | None
     out = torch.empty_like(x)
     shared_out = torch.empty_like(x) if L.shared_id >= 0 else None
     whole = x.shape[0] > s.rows and (pick is not None or gate is not None) and s.one_slot and _whole_prompt(x, L, gate)
-    step = min(WINDOWS_PROMPT_ROWS, _listed_rows(L)) if whole else s.rows
+    step = pass_rows(L, s.slots, WINDOWS_PROMPT_ROWS) if whole else s.rows
     for r0 in range(0, x.shape[0], step):
         rows = slice(r0, r0 + step)
         args = x[rows], None if pick is None else pick[rows], None if wts is None else wts[rows], L
@@ -505,12 +509,11 @@ class PrefillScratch:
 
 _PREFILL: dict = {}
 _PREFILL_KEPT: list = []     # outgrown prompt scratches that a captured graph may write to
-TILE_LIST_PAIRS = 32768      # esp_tile_list's limit on (expert slot, member tile) pairs
 
 
 def tile_list_cap(maxu: int, maxm: int, P: int, rows: int = 32) -> int:
-    """Entries esp_tile_list may write for a grouping of P picks over maxu expert slots, maxm members a row, in tiles of
-    `rows` members."""
+    """Entries esp_group_tiles (or esp_tile_list) may write for a grouping of P picks over maxu expert slots, maxm members
+    a row, in tiles of `rows` members."""
     return min(maxu * -(-maxm // rows), -(-P // rows) + maxu)
 
 
@@ -523,7 +526,9 @@ def tile_rows(T: int, k: int, E: int) -> int:
 
 
 def prefill_scratch(layer: Layer, rows: int, slots: int, device) -> PrefillScratch:
-    """The PrefillScratch shared by every layer of this layer's shape, for prompts of up to `rows` tokens."""
+    """The PrefillScratch shared by every layer of this layer's shape, for prompts of up to `rows` tokens, or of any number
+    from the tokens of one pass on (prefill's chunks)."""
+    rows = min(rows, pass_rows(layer, slots, PREFILL_MAX_ROWS))
     key = (layer.E, layer.D, layer.I, slots, str(device))
     found = _PREFILL.get(key)
     if found is None or found.rows < rows:
@@ -541,13 +546,13 @@ def prefill(x: torch.Tensor, pick: torch.Tensor | None, wts: torch.Tensor | None
             out_shared: torch.Tensor | None = None):
     """The MoE layer over a whole prompt (ESPALIER_PREFILL_MODE=tile): the picks of every token (vLLM's, or route_rows
     over the whole prompt, the bits decode's route_group gives them), ONE grouping of all of them, and the expert GEMMs
-    over that grouping with one K split, so each picked expert's weights are decoded once for all its member rows
-    (in tiles of 32) instead of once a 32-token window. Returns (routed sum, shared output or None), [T, D] in x's
+    over that grouping with one K split, so each picked expert's weights are decoded once for 32 or 64 of its member rows
+    (tile_rows) instead of once a 32-token window. Returns (routed sum, shared output or None), [T, D] in x's
     dtype; a token's output depends on its own picks and rows only (the K split is fixed), not on the other tokens.
-    A prompt of more than PREFILL_MAX_ROWS tokens, or of more (expert, 32-token tile) pairs than a tile list holds, runs as
-    consecutive chunks (the same bits a row)."""
+    A prompt of more tokens than one pass takes (pass_rows of PREFILL_MAX_ROWS) runs as consecutive chunks (the same bits a
+    row)."""
     T = x.shape[0]
-    step = min(PREFILL_MAX_ROWS, _listed_rows(L))
+    step = pass_rows(L, s.slots, PREFILL_MAX_ROWS)
     if T <= step:
         return _prefill(x, pick, wts, L, s, k, gate, out, out_shared)
     out = torch.empty((T, L.D), dtype=x.dtype, device=x.device) if out is None else out

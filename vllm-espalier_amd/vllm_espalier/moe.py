@@ -157,8 +157,7 @@ def run_grouped(L: grouped.Layer, x: torch.Tensor, pick, wts, k: int, router_wei
             grouped.route(x, router_weight, k, L, s)
         return grouped.routed2(x, pick, wts, L, s, k=k)
     if prefill_mode() == "tile":
-        return grouped.prefill(x, pick, wts, L, grouped.prefill_scratch(L, min(T, grouped.PREFILL_MAX_ROWS), slots,
-                                                                        x.device), k, gate=router_weight)
+        return grouped.prefill(x, pick, wts, L, grouped.prefill_scratch(L, T, slots, x.device), k, gate=router_weight)
     return grouped.windows(x, pick, wts, L, grouped.scratch(L, GROUPED_ROWS, slots, x.device), k=k,
                            gate=router_weight)
 
