@@ -1,4 +1,4 @@
-"""The whole-prompt expert launches (esp_grouped_prompt over esp_tile_list_rows): windows' tokens bit for bit those of the
+"""The whole-prompt expert launches (esp_grouped_prompt over esp_group_tiles' list): windows' tokens bit for bit those of the
 32-row window launches, at K splits of 4, 6 and 8 steps, tiles of 32 and 64 members, one to four row groups."""
 import pytest
 import torch

@@ -45,8 +45,9 @@ def test_group_wide_bit_exact(dev, ext, R, slots, E, maxm, repeats):
 
 
 def test_group_shared_wide_tables_equal_small(dev, ext):
-    """130 rows (1170 picks: the wide path) against the same rows in windows of 100 (the one-workgroup path): the pick
-    and weight tables bit for bit, the shared slot's sigmoid weight included; the grouping against the oracle."""
+    """130 rows (1170 picks) and 100 (900: a workgroup an id too, past 32 rows) against the same rows in windows of 30 (the
+    one-workgroup path): the pick and weight tables bit for bit, the shared slot's sigmoid weight included; the grouping
+    against the oracle."""
     gen = torch.Generator().manual_seed(5)
     R, k, E = 130, 8, 257
     pick = torch.stack([torch.randperm(256, generator=gen)[:k] for _ in range(R)]).to(torch.int32).to(dev)
@@ -66,13 +67,14 @@ def test_group_shared_wide_tables_equal_small(dev, ext):
         ext.group_shared(pick[r0:r1].contiguous(), wts[r0:r1].contiguous(), x[r0:r1], D, gw, 256, po, wo, uids,
                          count, members, r1 - r0, k, E)
         return po, wo, uids, count, members
-    po, wo, uids, count, members = tables(0, R)
-    a = tables(0, 100)
-    b = tables(100, R)
-    assert torch.equal(po, torch.cat([a[0], b[0]])) and torch.equal(wo, torch.cat([a[1], b[1]]))
-    cnt, u, m = O.group(po.cpu().numpy(), R, slots, E, R)
-    assert int(count.item()) == cnt
-    assert np.array_equal(uids[:cnt].cpu().numpy(), u) and np.array_equal(members[:cnt].cpu().numpy(), m)
+    few = [tables(r, min(r + 30, R)) for r in range(0, R, 30)]
+    for rows in (R, 100):
+        po, wo, uids, count, members = tables(0, rows)
+        n = rows * slots
+        assert torch.equal(po, torch.cat([t[0] for t in few])[:n]) and torch.equal(wo, torch.cat([t[1] for t in few])[:n])
+        cnt, u, m = O.group(po.cpu().numpy(), rows, slots, E, rows)
+        assert int(count.item()) == cnt
+        assert np.array_equal(uids[:cnt].cpu().numpy(), u) and np.array_equal(members[:cnt].cpu().numpy(), m)
 
 
 def _layer(n_experts, seed, dev):

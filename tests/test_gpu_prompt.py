@@ -77,16 +77,34 @@ def test_prompt_signed_zeros(dev):
     assert torch.equal(d.forward_prompt(x).view(torch.int16), _windows(d, x).view(torch.int16))
 
 
-@pytest.mark.parametrize("name", ["uneven_slots", "two_steps", "one_step", "one_split"])
+def _hows(d, T):
+    return [how for *_, how in d._tiles(T)]
+
+
+@pytest.mark.parametrize("name", ["uneven_slots", "two_steps", "one_step"])
 def test_tile_mode_rows_alone_equal_prompt(dev, name):
     """forward_tile past its rule runs as esp_dense_prompt: its rows alone (esp_dense_tile) have the same bits."""
     d = _layer(name, dev)
     T = 2100
+    assert _hows(d, T) == ["once"] and _hows(d, 1) == _hows(d, 128) == ["tile"]
     x = _rows(T, d.K, torch.bfloat16, dev, 8)
     y = d.forward_tile(x)
     for r in (0, 63, 64, 1000, 2099):
         assert torch.equal(d.forward_tile(x[r:r + 1]), y[r:r + 1]), r
     assert torch.equal(d.forward_tile(x[128:256]), y[128:256])
+
+
+@pytest.mark.parametrize("name", ["one_split", "nine_blocks"])
+def test_prompt_in_tile_order_equals_tile(dev, name):
+    """esp_dense_prompt at esp_dense_tile's sums (its K splits, two k slots), on layers too small for the rule to take it."""
+    d = _layer(name, dev)
+    T = 300
+    assert _hows(d, T) == ["tile"]
+    x = _rows(T, d.K, torch.bfloat16, dev, 8)
+    l, y = d.launches[0], torch.empty((T, d.n_out), dtype=x.dtype, device=dev)
+    d._prompt(x, [m.trellis for m in d.mats], [m.suh for m in d.mats], [m.svh for m in d.mats], y, l, D.tile_plan(d.K, l.n),
+              D.TILE_SLOTS)
+    assert torch.equal(y, d.forward_tile(x))
 
 
 def test_prompt_graph_replay(dev):
