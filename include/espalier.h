@@ -216,11 +216,8 @@ int esp_grouped_list(const void* X0, const void* X1, const int64_t* TP0, const i
                      int64_t z_numel, int64_t mats, int64_t K, int64_t N, int64_t P, int64_t SK, int64_t slots,
                      int64_t warps, int64_t lo, int64_t hi, void* stream);
 
-/* esp_tile_list for tiles of `rows` members (32 or 64): ceil(maxm / rows) and ceil(P / rows) in its bounds. */
-int esp_tile_list_rows(const int32_t* ucount, const int32_t* members, int64_t nexp_max, int64_t maxm, int64_t P,
-                       int64_t rows, int32_t* tiles, int64_t tiles_numel, void* stream);
-
-/* esp_group and esp_tile_list_rows of a whole prompt in one launch (no reference counterpart): the same tables, except
+/* esp_group of a whole prompt and its tile list for tiles of `rows` members (32 or 64; esp_tile_list's order, with
+ * ceil(maxm / rows) and ceil(P / rows) in its bounds) in one launch (no reference counterpart): the same tables, except
  * that a member row is filled with -1 to a whole tile only. maxm at most 11264. */
 int esp_group_tiles(const int32_t* pick, int32_t* uids, int64_t maxu, int32_t* ucount, int32_t* members, int64_t maxm,
                     int64_t R, int64_t slots, int64_t E, int64_t rows, int32_t* tiles, int64_t tiles_numel, void* stream);
@@ -230,7 +227,7 @@ int esp_shared_slots(const int32_t* pick_in, const float* wts_in, const void* x,
                      const void* gate_w, int64_t shared_id, int32_t* pick_out, float* wts_out, int64_t R,
                      int64_t slots_in, void* stream);
 
-/* The expert GEMMs of a whole prompt over esp_tile_list_rows's list for tiles of tile_rows members (no reference
+/* The expert GEMMs of a whole prompt over esp_group_tiles' list for tiles of tile_rows members (no reference
  * counterpart): an expert's weights decoded once a tile and matrix, every split's scaled sums added in split order in
  * the launch, so Z [mats][P][N] holds what esp_grouped's readers make of its [mats][SK][P][N] at SK splits and one wave
  * of k slots (4 waves a workgroup), bit for bit. K and N multiples of 128, P * K < 2^31. Status bits as esp_grouped and

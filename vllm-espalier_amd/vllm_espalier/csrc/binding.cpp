@@ -61,17 +61,15 @@ void grouped(const at::Tensor& X0, const at::Tensor& X1, const at::Tensor& TP0, 
                      K, N, P, SK, slots, nt, warps, pf, lo, hi, cur_stream()));
 }
 
-// esp_tile_list_rows: the non-empty (expert slot, member tile) pairs of a grouping, for grouped_list (tiles of 32
-// members) and grouped_prompt (32 or 64)
-void tile_list(const at::Tensor& ucount, const at::Tensor& members, int64_t nexp_max, int64_t P, at::Tensor tiles,
-               int64_t rows) {
+// esp_tile_list: the non-empty (expert slot, member tile) pairs of a grouping, for grouped_list
+void tile_list(const at::Tensor& ucount, const at::Tensor& members, int64_t nexp_max, int64_t P, at::Tensor tiles) {
     check(ucount, at::kInt, "ucount");
     check(members, at::kInt, "members");
     check(tiles, at::kInt, "tiles");
     TORCH_CHECK(members.dim() == 2 && members.size(0) >= nexp_max, "members: [nexp_max, maxm]");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(members.device());
-    call(esp_tile_list_rows(cptr<int32_t>(ucount), cptr<int32_t>(members), nexp_max, members.size(1), P, rows,
-                            mptr<int32_t>(tiles), tiles.numel(), cur_stream()));
+    call(esp_tile_list(cptr<int32_t>(ucount), cptr<int32_t>(members), nexp_max, members.size(1), P,
+                       mptr<int32_t>(tiles), tiles.numel(), cur_stream()));
 }
 
 // esp_grouped_list: grouped's programs over tile_list's entries only (the same bits)
@@ -103,7 +101,7 @@ void grouped_list(const at::Tensor& X0, const at::Tensor& X1, const at::Tensor& 
                           mptr<float>(Z), Z.numel(), mats, K, N, P, SK, slots, warps, lo, hi, cur_stream()));
 }
 
-// esp_grouped_prompt: the experts of a whole prompt over tile_list's entries, one partial a row with the bits of grouped
+// esp_grouped_prompt: the experts of a whole prompt over group_tiles' list, one partial a row with the bits of grouped
 // at SK splits and their sum
 void grouped_prompt(const at::Tensor& X0, const at::Tensor& X1, const at::Tensor& TP0, const at::Tensor& TP1,
                     const at::Tensor& B0, const at::Tensor& B1, const at::Tensor& C0, const at::Tensor& C1,
@@ -832,8 +830,7 @@ PYBIND11_MODULE(espalier_ext, m) {
     m.def("group_shared", &group_shared);
     m.def("down_combine2", &down_combine2);
     m.def("grouped", &grouped);
-    m.def("tile_list", &tile_list, py::arg("ucount"), py::arg("members"), py::arg("nexp_max"), py::arg("P"),
-          py::arg("tiles"), py::arg("rows") = 32);
+    m.def("tile_list", &tile_list);
     m.def("grouped_prompt", &grouped_prompt);
     m.def("group_tiles", &group_tiles);
     m.def("shared_slots", &shared_slots);

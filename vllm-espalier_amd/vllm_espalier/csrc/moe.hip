@@ -1162,7 +1162,7 @@ __global__ __launch_bounds__(64) void down_combine_rows_kernel(const float* __re
 
 // ------------------------------------------------------------------------------------------------------------------
 // esp_tile_list: the non-empty (expert slot u, member tile t) pairs of a grouping, in (u, t) order, for
-// esp_grouped_list (tiles of 32 members) and esp_grouped_prompt (32 or 64): tiles[0] = their number, tiles[1 + i] = u << 16 | t. A tile is non-empty iff its first member is
+// esp_grouped_list: tiles[0] = their number, tiles[1 + i] = u << 16 | t. A tile is non-empty iff its first member is
 // (members come first in a row, -1 padded). One workgroup: each thread tests its run of consecutive pairs with every
 // load in flight, then a block-wide prefix of the counts places the entries. At most cap entries are written; a
 // grouping with more raises ESP_STATUS_TILE_LIST (its grouped launches would miss tiles).
@@ -1171,7 +1171,7 @@ constexpr int TL_THREADS = 1024, TL_PER = 32;           // pairs a thread at mos
 
 __global__ __launch_bounds__(TL_THREADS) void tile_list_kernel(const int* __restrict__ ucount,
                                                               const int* __restrict__ members, int maxu, int maxm,
-                                                              int mt, int rows, int* __restrict__ tiles, int cap) {
+                                                              int mt, int* __restrict__ tiles, int cap) {
     __shared__ int wave_tot[TL_THREADS / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // the count and the first eight pairs' first members in flight together: every slot of the member table lies
@@ -1188,7 +1188,7 @@ __global__ __launch_bounds__(TL_THREADS) void tile_list_kernel(const int* __rest
             v[i] = -1;
             if (i0 + i < per && q < maxu * mt) {
                 const int u = q / mt, t = q - u * mt;
-                v[i] = members[(size_t)u * maxm + t * rows];
+                v[i] = members[(size_t)u * maxm + t * 32];
             }
         }
         if (pairs < 0) {
@@ -2137,7 +2137,7 @@ extern "C" int esp_group_tiles(const int32_t* pick, int32_t* uids, int64_t maxu,
     ESP_REQUIRE(R >= 1 && R * slots <= (int64_t(1) << 24), "grouping window too large");
     ESP_REQUIRE(maxu >= (R * slots < E ? R * slots : E), "uids too small");
     ESP_REQUIRE(maxm >= 1 && maxm <= 11264, "group_tiles: at most 11264 members an expert");      // 44 KiB beside the counts
-    ESP_REQUIRE(rows == 32 || rows == 64, "tile_list: tiles of 32 or 64 members");
+    ESP_REQUIRE(rows == 32 || rows == 64, "group_tiles: tiles of 32 or 64 members");
     const int64_t cap = tile_list_cap(R * slots < E ? R * slots : E, maxm, R * slots, rows);
     ESP_REQUIRE(tiles_numel >= 1 + cap, "group_tiles: tiles needs 1 + min(U * ceil(maxm / rows), ceil(P / rows) + U) ints "
                                         "(P = R * slots picks, U = min(P, E) expert slots)");
@@ -2163,24 +2163,17 @@ extern "C" int esp_shared_slots(const int32_t* pick_in, const float* wts_in, con
     return esp_host::launch_check("shared_slots");
 }
 
-extern "C" int esp_tile_list_rows(const int32_t* ucount, const int32_t* members, int64_t nexp_max, int64_t maxm,
-                                  int64_t P, int64_t rows, int32_t* tiles, int64_t tiles_numel, void* stream) {
+extern "C" int esp_tile_list(const int32_t* ucount, const int32_t* members, int64_t nexp_max, int64_t maxm, int64_t P,
+                             int32_t* tiles, int64_t tiles_numel, void* stream) {
     ESP_REQUIRE(ucount && members && tiles, "tile_list: null pointer");
     ESP_REQUIRE(nexp_max >= 1 && nexp_max < 65536 && maxm >= 1 && maxm <= 65536 && P >= 1,
                 "tile_list: 1 to 65535 expert slots, 1 to 65536 members a row, P >= 1");
-    ESP_REQUIRE(rows == 32 || rows == 64, "tile_list: tiles of 32 or 64 members");
-    const int64_t mt = (maxm + rows - 1) / rows, cap = tile_list_cap(nexp_max, maxm, P, rows);
+    const int64_t mt = (maxm + 31) / 32, cap = tile_list_cap(nexp_max, maxm, P);
     ESP_REQUIRE(nexp_max * mt <= (int64_t)TL_THREADS * TL_PER, "tile_list: at most 32768 (expert, member tile) pairs");
-    ESP_REQUIRE(tiles_numel >= 1 + cap,
-                "tile_list: tiles needs 1 + min(E * ceil(maxm / rows), ceil(P / rows) + E) ints (rows a tile)");
+    ESP_REQUIRE(tiles_numel >= 1 + cap, "tile_list: tiles needs 1 + min(E * ceil(maxm / 32), ceil(P / 32) + E) ints");
     tile_list_kernel<<<1, TL_THREADS, 0, (hipStream_t)stream>>>(ucount, members, (int)nexp_max, (int)maxm, (int)mt,
-                                                                (int)rows, tiles, (int)cap);
+                                                                tiles, (int)cap);
     return esp_host::launch_check("tile_list");
-}
-
-extern "C" int esp_tile_list(const int32_t* ucount, const int32_t* members, int64_t nexp_max, int64_t maxm, int64_t P,
-                             int32_t* tiles, int64_t tiles_numel, void* stream) {
-    return esp_tile_list_rows(ucount, members, nexp_max, maxm, P, 32, tiles, tiles_numel, stream);
 }
 
 extern "C" int esp_grouped_list(const void* X0, const void* X1, const int64_t* TP0, const int64_t* TP1,

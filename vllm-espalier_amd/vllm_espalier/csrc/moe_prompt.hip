@@ -20,7 +20,7 @@ struct GroupedPromptArgs {
     const int* uids;
     const int* ucount;
     const int* members;
-    const int* tiles;              // tile_list_kernel's list for tiles of TR members
+    const int* tiles;              // esp_group_tiles' list for tiles of TR members
     float* Z;                      // [mats][P][N]
     int K, N, P, maxm, slots;
     int split_steps;               // 32-k steps of a split

@@ -51,7 +51,7 @@ FUSED_ROWS = 4
 # (esp_moe_chain: the down programs decode their weights while gate/up runs; the same bits); ESPALIER_MOE_CHAIN=0 off
 CHAIN = env("ESPALIER_MOE_CHAIN", "1") != "0"
 CHAIN_ROWS = 4
-PREFILL_WAVES = 4          # waves a workgroup of the whole-prompt grouped launches
+PREFILL_WAVES = 4          # waves a workgroup of esp_grouped_list over a whole prompt (prefill runs esp_grouped_prompt)
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 
