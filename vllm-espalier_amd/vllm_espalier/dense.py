@@ -18,7 +18,7 @@ from dataclasses import dataclass, field
 import torch
 
 from ._env import env
-from ._streams import hand_out
+from ._streams import hand_out, raw_stream
 from .experts import KERNEL_CB, ext
 
 MAX_ROWS = 32
@@ -116,12 +116,12 @@ class _SharedScratch:
 
     def reserve(self, device, z_floats: int, xh_halves: int):
         have = self.current.get(device)
-        capturing = device.type == "cuda" and torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
+        capturing = device.type == "cuda" and torch.cuda.is_current_stream_capturing()
         if have is not None and have[0].numel() >= z_floats and have[1].numel() >= xh_halves:
             if capturing:
                 self.captured.add(device)
-            else:
-                hand_out(have, self.streams[device], device)
+            elif (raw := raw_stream(device)) not in self.streams[device]:
+                hand_out(have, self.streams[device], device, raw)
             return have
         if have is not None:
             if device in self.captured:
@@ -133,7 +133,7 @@ class _SharedScratch:
             z.fill_(self.fill)
         pair = (z.view(self.dtype), torch.empty(max(xh_halves, 1), dtype=torch.float16, device=device))
         self.current[device] = pair
-        self.streams[device] = set()
+        self.streams[device] = {raw_stream(device)}
         if capturing:
             self.captured.add(device)
         return pair

@@ -33,7 +33,7 @@ from pathlib import Path
 import torch
 
 from ._env import env
-from ._streams import hand_out
+from ._streams import hand_out, raw_stream
 
 # Espalier grid code (EspMatrix.cb) -> the kernels' codebook id (exllamav3's: 1 mcg, 3 E2M1, 6 int5, 7 int6)
 KERNEL_CB = {0: 1, 1: 3, 3: 6, 4: 7}
@@ -477,7 +477,7 @@ class PrefillScratch:
     def __init__(self, E: int, D: int, I: int, rows: int, slots: int, device, window: int = 32):
         self.rows, self.slots, self.E, self.window = rows, slots, E, window
         self.captured = False                            # handed out during a graph capture
-        self.streams: set = set()                        # streams that its buffers are recorded on
+        self.streams: set = {raw_stream(torch.device(device))}   # streams that its buffers are recorded on, and their own
         P = rows * slots
         maxu = min(P, E)
         f16, f32, i32 = torch.float16, torch.float32, torch.int32
@@ -496,10 +496,11 @@ class PrefillScratch:
     def handed_out(self) -> PrefillScratch:
         """Note a use on the current stream: a captured one makes whoever replaces this scratch keep it, another holds its
         memory until that stream is done with it."""
-        if torch.cuda.is_available() and torch.cuda.is_current_stream_capturing():
+        device = self.z.device
+        if device.type == "cuda" and torch.cuda.is_current_stream_capturing():
             self.captured = True
-        else:
-            hand_out(self.tensors, self.streams, self.z.device)
+        elif (raw := raw_stream(device)) not in self.streams:
+            hand_out(self.tensors, self.streams, device, raw)
         return self
 
     def grouping(self, T: int):
