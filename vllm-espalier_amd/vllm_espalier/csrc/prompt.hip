@@ -182,10 +182,12 @@ __device__ __forceinline__ void wait_vm_lgkm0() {
 // copies a step (row groups past the prompt and steps past the last are clamped, read and not used), so the counts hold.
 //
 // SPS > 0: every split is 4 slots of SPS steps (the plans of narrow layers), a loop iteration whose slots the compiler
-// knows; 0: any order, counted down at run time.
+// knows; 0: any order, counted down at run time, at the price of 20 spilled registers, which come back at each split's end:
+// the wait for them there also drains the copies in flight.
 //
-// Bound by the shared memory's bandwidth (12 KiB written and 24 KiB read a step, ~290 clocks against 128 of MFMA), hidden
-// by three workgroups a CU where the grid holds them. A 128-row tile halves the B reads a row, but its three sets of
+// Bound by the shared memory: 12 KiB written and 24 KiB read a step are ~290 clocks of its bandwidth against 128 of MFMA, so
+// at most 44 % of the matrix peak, of which 30 % are reached at 2048 rows of 2048 -> 5120 (58 us); the reads' latency is
+// hidden by three workgroups a CU where the grid holds them. A 128-row tile halves the B reads a row, but its three sets of
 // sums (slot, split, total: 192 registers) leave two waves a SIMD: 2048 x 2048 -> 5120, 94 us against 58.
 template <int SPS>
 __global__ __launch_bounds__(PG_WAVES * 64, 3) void prompt_gemm_kernel(PromptArgs a) {
