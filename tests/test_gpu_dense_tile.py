@@ -209,7 +209,7 @@ def test_outgrown_prompt_scratch_outlives_its_streams(dev, monkeypatch):
     a.synchronize()
     b.wait_stream(a)
     with torch.cuda.stream(b):
-        torch.cuda._sleep(20_000_000)
+        torch.cuda._sleep(400_000_000)                     # ~0.17 s
         got = d.forward_tile(x)
         d.forward_tile(longer)                                # drops the first scratch
     assert [t.data_ptr() for t in D.prompt_scratch(dev, 0, 0, 0)] != [p for p, _ in first]

@@ -154,7 +154,7 @@ def test_outgrown_prompt_scratch_outlives_its_streams(dev, mode):
     a.synchronize()
     b.wait_stream(a)
     with torch.cuda.stream(b):
-        torch.cuda._sleep(20_000_000)
+        torch.cuda._sleep(400_000_000)                     # ~0.17 s
         got = run(x)
         run(longer)                                           # drops the first scratch
     with torch.cuda.stream(a):
